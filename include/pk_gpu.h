@@ -425,8 +425,9 @@ void pk_gpu_encoder_destroy(pk_gpu_encoder *enc);
 int pk_gpu_num_configs(void);
 int pk_gpu_config_info(int index, int *family, int *mfma, int *cw, int *wgm, int *wgn,
                        int *kt);
-/* Index of the configuration the dispatcher picks for a shape with int8
- * weights, and for weights of `bits` = 4, 8 or 32 (fp32) bits (-1 for any
+/* Index of the configuration that the K = 1 chain kernels take (forced
+ * configurations, alpha other than 1, unaligned operands) for a shape with
+ * int8 weights, and for weights of `bits` = 4, 8 or 32 (fp32) bits (-1 for any
  * other value). */
 int pk_gpu_pick_config(int M, int N, int K);
 int pk_gpu_pick_config_bits(int M, int N, int K, int bits);
@@ -569,6 +570,14 @@ int pk_gpu_force_panel_tile(int mb, int nct);
  * encoder runs included: an encoder keeps its captured graphs per forced
  * configuration, so a change takes effect on the next run. */
 int pk_gpu_force_config(int index);
+
+/* The exact GEMMs' own tiles (16-byte aligned rows, alpha = 1): their number,
+ * the one that a shape with weights of `bits` = 4, 8 or 32 bits takes (-1:
+ * invalid), and a test hook that forces one for later GEMM calls on this
+ * thread (-1 = automatic).  The tile never changes a result. */
+int pk_gpu_num_chain_tiles(void);
+int pk_gpu_pick_chain_tile(int M, int N, int bits);
+int pk_gpu_force_chain_tile(int tile);
 
 #ifdef __cplusplus
 }

@@ -116,7 +116,9 @@ struct TileConfig {
     int threads() const { return (family == 'S' ? 128 : 64) * wgm * wgn; }
 };
 
-// Pick the tile configuration with the lowest modelled time on 256 CUs.
+// The configuration the K = 1 chain kernels take for a shape.  They run the
+// forced configurations and what the four-deep chains (pk_chain4.h) do not
+// take: alpha other than 1, and operands whose rows allow no vector loads.
 int choose_config_index(int M, int N, int K, WeightKind kind);
 // Number of configurations and access by index (for tests and sweeps).
 int num_configs();

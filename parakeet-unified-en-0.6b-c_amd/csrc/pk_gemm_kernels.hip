@@ -1,6 +1,8 @@
 // pk_gemm_kernels.hip - dispatch of the weight GEMMs and the small kernels
 // around them (beta-only pass, int8 edge columns, swish).  The tile kernels
 // and their numerics are described in pk_gemm_tiles.h.
+#include "pk_chain4.h"
+#include "pk_gpu.h"
 #include "pk_gemm_tiles.h"
 
 namespace pkgpu {
@@ -101,6 +103,42 @@ static int choose_index(int M, int N, int K, WeightKind kind = W_I8)
 
 int choose_config_index(int M, int N, int K, WeightKind kind) { return choose_index(M, N, K, kind); }
 
+namespace {
+// us for the first round of workgroups (one on every CU) and for each further
+// one at K = 1024, by weight format and tile (pk_chain4.h).  Fitted to all
+// tiles at M = 1..3312 over N = 1024..4096 and K = 1024, 4096 on MI355X; K
+// scales all of a row alike.  A CU's workgroups share its matrix cores, so a
+// further round costs its MFMAs, and the first one also the time that one
+// workgroup alone leaves them idle.  The 16 x 32 tile is the fastest until a
+// second round, 128 x 64 from about 20 outputs per thread of the chip on.
+struct Rounds { float first, next; };
+constexpr Rounds kChain4Rounds[3][chain4::kNumTiles] = {
+    /* fp32 */ {{6.5f, 3.8f}, {7.0f, 4.1f}, {10.3f, 7.4f}, {11.2f, 7.9f}, {18.6f, 16.2f}, {35.2f, 31.0f}},
+    /* int8 */ {{6.8f, 4.0f}, {9.5f, 4.6f}, {11.3f, 8.0f}, {13.8f, 9.0f}, {24.3f, 15.7f}, {40.6f, 32.0f}},
+    /* int4 */ {{6.7f, 4.5f}, {9.2f, 4.7f}, {10.7f, 7.6f}, {13.4f, 8.9f}, {22.9f, 16.8f}, {38.7f, 32.5f}},
+};
+constexpr int kCus = 256;
+thread_local int t_chain_tile = -1;
+
+int chain4_pick(int M, int N, WeightKind kind)
+{
+    int best = 0;
+    double best_t = 0.0;
+    for (int i = 0; i < chain4::kNumTiles; ++i) {
+        const chain4::Chain4Tile& t = chain4::kTiles[i];
+        const long long wgs = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const Rounds& r = kChain4Rounds[kind][i];
+        const double time = r.first + r.next * (double)((wgs + kCus - 1) / kCus - 1);
+        if (i == 0 || time < best_t) {
+            best = i;
+            best_t = time;
+        }
+    }
+    return best;
+}
+}  // namespace
+
+
 hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, Tolerance tol)
 {
     if (p.M <= 0 || p.N <= 0) return hipSuccess;
@@ -195,10 +233,21 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, 
     if (p.kind == W_I8) n_main = (p.N / 16) * 16;     // blas.c:686, 734
     a.N = n_main;
 
-    const int cfg = (cfg_index >= 0 && cfg_index < kNumConfigs) ? cfg_index
-                                                                : choose_index(p.M, n_main, p.K, p.kind);
     hipError_t err = hipSuccess;
-    if (n_main > 0) {
+    if (n_main > 0 && cfg_index < 0 && a.vec_a && a.vec_b && a.alpha == 1.0f) {
+        // The four-deep chains: the same bits, faster at every size measured.
+        // They read whole vectors and take A as it is; other operands stay on
+        // the K = 1 tiles.
+        const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.kind);
+        switch (p.kind) {
+        case W_F32: err = chain4::launch_f32(tile, a, stream); break;
+        case W_I8:  err = chain4::launch_i8(tile, a, stream); break;
+        case W_I4:  err = chain4::launch_i4(tile, a, stream); break;
+        }
+        if (err != hipSuccess) return err;
+    } else if (n_main > 0) {
+        const int cfg = (cfg_index >= 0 && cfg_index < kNumConfigs) ? cfg_index
+                                                                    : choose_index(p.M, n_main, p.K, p.kind);
         switch (p.kind) {
         case W_F32: err = tiles::launch_chain_f32(cfg, a, stream); break;
         case W_I8:  err = tiles::launch_chain_i8(cfg, a, stream); break;
@@ -282,3 +331,27 @@ hipError_t launch_swish(const float* x, float* y, long long n, hipStream_t strea
 }
 
 }  // namespace pkgpu
+
+extern "C" {
+
+int pk_gpu_num_chain_tiles(void) { return pkgpu::chain4::kNumTiles; }
+
+int pk_gpu_pick_chain_tile(int M, int N, int bits)
+{
+    if (M <= 0 || N <= 0) return -1;
+    switch (bits) {
+    case 4: return pkgpu::chain4_pick(M, N, pkgpu::W_I4);
+    case 8: return pkgpu::chain4_pick(M, N, pkgpu::W_I8);
+    case 32: return pkgpu::chain4_pick(M, N, pkgpu::W_F32);
+    default: return -1;
+    }
+}
+
+int pk_gpu_force_chain_tile(int tile)
+{
+    if (tile >= pkgpu::chain4::kNumTiles) return PK_GPU_EINVAL;
+    pkgpu::t_chain_tile = tile < 0 ? -1 : tile;
+    return PK_GPU_OK;
+}
+
+}  // extern "C"
