@@ -7,37 +7,29 @@
 
 namespace pkgpu {
 
-// Longest chunk whose score rows the attention kernel keeps in LDS.  The
-// reference's encoder never attends over more than 500 frames unless
-// chunking is forced off (PK_CHUNK_THRESHOLD, parakeet.h; encoder.c:595-610);
-// longer sequences keep each workgroup's score rows in a device workspace
-// (AttnArgs::scores) and run the same arithmetic.
+// Longest chunk that attends without a workspace.  The reference's encoder
+// never attends over more than 500 frames unless chunking is forced off
+// (PK_CHUNK_THRESHOLD, parakeet.h; encoder.c:595-610); for longer sequences the
+// caller gives AttnArgs::scores, which holds the score rows that LDS does not.
 constexpr int kAttnMaxT = 512;
-constexpr int kAttnRows = 32;          // query rows per workgroup
-// LDS row stride of a workgroup's score rows for chunks of T rows, and the
-// workgroup's LDS: the score rows plus one staging tile of 64 x 68 floats.
-// The stride is 8 more than a multiple of 32 floats, so rows 8 apart in
-// banks: the softmax's 4 rows x 8 lanes and the value loop's 4 rows x 8
-// keys per half wave reach 32 distinct banks.  At T = 416 two workgroups
-// fit in a CU's 160 KiB.
+constexpr int kAttnRows = 32;          // query rows per workgroup (fast and long)
+// Row stride of a workgroup's score rows in that workspace, and in the fast
+// attention's LDS.
 __host__ __device__ constexpr int attn_sld(int T) { return ((T + 31) & ~31) + 8; }
-__host__ __device__ constexpr unsigned attn_lds_bytes(int T)
+// Row stride of the exact attention's score rows in LDS: 4 more than a multiple
+// of 32 floats, so that the 4 x 16 scores a wave instruction stores (rows 4
+// apart) reach every bank twice, and the softmax's 4 rows x 16 lanes nearly so.
+__host__ __device__ constexpr int attn4_sld(int T) { return ((T + 31) & ~31) + 4; }
+// LDS of its workgroup of 16 rt rows and nw waves (160 KB in a CU): the score
+// rows and, staged, 16 rows of 132 floats per wave and for each 16 rows of Q.
+constexpr int kLdsBytes = 160 * 1024;
+constexpr size_t attn_lds_bytes(int T, int rt, int nw, bool stage)
 {
-    return 4u * (unsigned)(kAttnRows * attn_sld(T) + 64 * 68);
+    return 4u * ((stage ? (size_t)(rt + nw) * 16 * 132 : 0) + (size_t)16 * rt * attn4_sld(T));
 }
 
-// Sequences of at most kAttnShortT rows take rel_pos_attention_short:
-// kAttnShortRows query rows per workgroup, and every key, position and value
-// row it reads staged in LDS at once (the score rows, then 64 key rows, one
-// or two blocks of 64 position rows and the value rows, T rounded up to 16,
-// each kTileLd = 132 floats apart).
+// Sequences of at most kAttnShortT rows never take the fast attention.
 constexpr int kAttnShortT = 64;
-constexpr int kAttnShortRows = 16;
-__host__ __device__ constexpr unsigned attn_short_lds_bytes(int T)
-{
-    return 4u * (unsigned)(kAttnShortRows * attn_sld(T) +
-                           (64 + 64 * ((T + kAttnShortRows - 1 + 63) / 64) + ((T + 15) & ~15)) * 132);
-}
 
 // Relative-position attention of n chunks (encoder.c:300-408); chunk z has
 // chunk_T[z] <= T rows (all T when chunk_T is null).

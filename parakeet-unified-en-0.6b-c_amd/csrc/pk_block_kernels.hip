@@ -25,6 +25,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <array>
 #include <utility>
 
 namespace pkgpu {
@@ -199,11 +200,15 @@ __global__ __launch_bounds__(256) void layer_norm_split_rows(const float* x, int
 }
 
 // ---- relative-position attention (encoder.c:300-408) ------------------------
-// One workgroup: 32 query rows of one head of one chunk, 4 waves of 8 rows.
-// Products use v_mfma_f32_4x4x1_16b_f32 with block 0's A broadcast to all 16
-// blocks (CBSZ = 4): one MFMA = 4 rows x 64 columns, lane j holds column j of
-// rows 0..3, and the A register lane 4t + i holds row i at k-step t (ABID =
-// t).  Each MFMA is one fused multiply-add per output.
+// rel_pos_attention4 multiplies on v_mfma_f32_16x16x4_f32, whose four products per
+// output are added one after another, each as a fused multiply-add (see
+// pk_chain4.h); rel_pos_attention_long (scores that do not fit in LDS) takes 32
+// query rows of one head by 4 waves of 8 rows on v_mfma_f32_4x4x1_16b_f32 with
+// block 0's A broadcast to all 16 blocks (CBSZ = 4): one MFMA = 4 rows x 64
+// columns, lane j holds column j of rows 0..3, and the A register lane 4t + i
+// holds row i at k-step t (ABID = t).  Measured, one sequence of 8 heads, us,
+// against the latter (with its scores in LDS up to T = 512): T = 33 9.0 -> 8.6,
+// 100 20.4 -> 12.3, 416 48.4 -> 23.5, 700 99.9 -> 58.1, 1101 220.7 -> 142.
 //
 // Scores (NT dot products, blas.c:221-249): eight accumulators per output,
 // step k goes to accumulator k % 8, so accumulator l is the chain over
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(256) void layer_norm_split_rows(const float* x, int
 constexpr int kDh = 128;                 // PK_HEAD_DIM
 constexpr int kTileLd = kDh + 4;         // padded LDS row of a value tile
 constexpr float kScoreScale = 0.0883883461356163f;   // 1/sqrtf(128) = 0x3db504f3
-static_assert(kTileLd == 132, "attn_short_lds_bytes counts staged rows of 132 floats");
+static_assert(kTileLd == 132, "attn_lds_bytes counts staged rows of 132 floats");
 
 template <int T_>
 __device__ inline v4f mfma_bcast(float a, float b, v4f c)
@@ -460,22 +465,395 @@ __device__ inline void softmax_row(float* s, int T, bool live)
     }
 }
 
-// kGlobal: the block's score rows live in its own slice of p.scores (task
-// order) instead of LDS, for sequences beyond kAttnMaxT; every operation and
-// its order are the same, and __syncthreads orders the workgroup's global
-// writes as it does its LDS writes.
-template <bool kGlobal>
-__global__ __launch_bounds__(256, 2) void rel_pos_attention(AttnArgs p)
+// Softmax of one score row s[0, T) in place (tensor_ops.c:336-357), by the 16
+// lanes of an aligned group: as softmax_row, whose lane q owns j = q, q + 8, ...,
+// with every second of its elements evaluated by lane q + 8 and added to lane
+// q's partial sum in the same order.
+__device__ inline void softmax_row16(float* s, int T)
 {
-    // Scores of the block's rows [kAttnRows][sld], then one staging tile.
+    const int lane = threadIdx.x & 63, q = lane & 15;
+    float mx = s[0];
+#pragma unroll 4
+    for (int j = q; j < T; j += 16) mx = fmaxf(mx, s[j]);
+    mx = fmaxf(mx, __shfl_xor(mx, 8));
+    mx = fmaxf(mx, __shfl_xor(mx, 4));
+    mx = fmaxf(mx, __shfl_xor(mx, 2));
+    mx = fmaxf(mx, __shfl_xor(mx, 1));
+    const int T8 = T & ~7, T16 = T & ~15;
+    float part = 0.0f;
+    auto group = [&](int j0, auto N) {                // 16 N elements
+        float e[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) e[n] = exp_poly(__fsub_rn(s[j0 + 16 * n + q], mx));
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            s[j0 + 16 * n + q] = e[n];
+            // lane q + 8's e, rotated into lane q of the row of 16
+            const float hi = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(e[n]), 0x128, 0xf, 0xf, true));
+            part = __fadd_rn(__fadd_rn(part, e[n]), hi);
+        }
+    };
+    int j0 = 0;
+    for (; j0 + 64 <= T16; j0 += 64) group(j0, std::integral_constant<int, 4>{});
+    for (; j0 < T16; j0 += 16) group(j0, std::integral_constant<int, 1>{});
+    if (T16 < T8 && q < 8) {
+        const float e = exp_poly(__fsub_rn(s[T16 + q], mx));
+        s[T16 + q] = e;
+        part = __fadd_rn(part, e);
+    }
+    float sum = hsum8_lanes(part);
+    if (T8 < T && q == 0)             // scalar tail, one lane, in order
+        for (int j = T8; j < T; ++j) {
+            const float e = expf_ieee(__fsub_rn(s[j], mx));
+            s[j] = e;
+            sum = __fadd_rn(sum, e);
+        }
+    sum = __shfl(sum, lane & ~15);
+    const float inv = __fdiv_rn(1.0f, sum);
+#pragma unroll 4
+    for (int j = q; j < T; j += 16) s[j] = __fmul_rn(s[j], inv);
+}
+
+// 16 rows of a score operand, read row by row (a wave instruction takes two
+// whole rows) and turned to the operand layout in an LDS buffer that only this
+// wave uses.  The layout itself, read from memory, is 64 pieces of 16 bytes an
+// instruction, and the CU's one address unit takes as long over them as the
+// matrix cores over a 16 x 16 block.
+constexpr int kScoreRows = 16 * kTileLd;
+struct ScoreRows {
+    v4f r[8];
+    // rows `row`.. past the descriptor's first one; a negative row or one past
+    // its range reads 0
+    __device__ void load(__amdgpu_buffer_rsrc_t rs, int row, int ld)
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            r[i] = __builtin_bit_cast(v4f, tiles::ld_v4(rs, ((uint32_t)(row + 2 * i + (lane >> 5)) * (uint32_t)ld +
+                                                             4u * (lane & 31)) * 4u));
+    }
+    __device__ void put(float* buf) const
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<v4f*>(buf + (2 * i + (lane >> 5)) * kTileLd + 4 * (lane & 31)) = r[i];
+        // the wave's own LDS accesses stay in this order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+};
+// The operand as v_mfma_f32_16x16x4_f32 takes it: lane j + 16 g holds columns
+// 32 i + 8 g + l (i < 4, l < 8) of row j.  Instruction (i, l) then multiplies
+// columns 32 i + l + {0, 8, 16, 24}, four consecutive steps of the chain l over
+// k = l, l + 8, ...
+struct ScoreRow {
+    v4f v[4][2];
+    __device__ float at(int i, int l) const { return v[i][l >> 2][l & 3]; }
+    // straight from memory; `row` as ScoreRows::load's
+    __device__ void load(__amdgpu_buffer_rsrc_t rs, int row, int ld)
+    {
+        const int lane = threadIdx.x & 63;
+        const uint32_t off = ((uint32_t)(row + (lane & 15)) * (uint32_t)ld + 8u * (lane >> 4)) * 4u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                v[i][h] = __builtin_bit_cast(v4f, tiles::ld_v4(rs, off + 4u * (32 * i + 4 * h)));
+    }
+    // from a wave's buffer
+    __device__ void get(const float* buf)
+    {
+        const int lane = threadIdx.x & 63;
+        const float* row = buf + (lane & 15) * kTileLd + 8 * (lane >> 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[i][h] = *reinterpret_cast<const v4f*>(row + 32 * i + 4 * h);
+    }
+};
+
+// One workgroup: 16 RT query rows of one head of one chunk, NW waves.
+// - AC = Q_u K^T: wave w takes blocks w, w + NW, ... of 16 keys, two blocks ahead
+//   from memory and one from its LDS buffer (no other wave reads them).  16 x 16
+//   scores are 8 chains of 4 instructions.
+// - BD = Q_v P^T: likewise over blocks of 16 positions, whose loads start while
+//   the last keys are multiplied; a score's column is j = m - (T-1-i), where it
+//   is added to AC and scaled.
+// - softmax, 16 lanes a row.
+// - scores x V: the chain over keys cannot be split, so each wave takes 128 / NW
+//   of the output columns, its values loaded 96 keys ahead.
+// kStage: keys, positions and Q go through LDS (see ScoreRows).  It costs
+// 8.4 KB a wave, and is taken where one workgroup a CU is all there is.
+template <int RT, int NW, bool kStage>
+__global__ __launch_bounds__(64 * NW, 2) void rel_pos_attention4(AttnArgs p)
+{
+    constexpr int ROWS = 16 * RT, CW = 8 / NW;
+    typedef float vcw __attribute__((ext_vector_type(CW)));
     extern __shared__ float smem[];
+    const int sld = attn4_sld(p.T);
+    int rb, h, z;
+    attn_task(rb, h, z);
+    // LDS: kStage: Q [ROWS][kTileLd] and the waves' buffers [NW][16][kTileLd];
+    // then the score rows
+    constexpr int kBase = kStage ? (RT + NW) * kScoreRows : 0;
+    float* Q = smem;
+    float* S = smem + kBase;
+    // this chunk's rows (the compiler loads them through a select of two
+    // addresses, into a vector register: descriptors need them uniform)
+    const int T = __builtin_amdgcn_readfirstlane(p.chunk_T ? p.chunk_T[z] : p.T);
+    const int r0 = rb * ROWS;
+    if (r0 >= T) return;                                     // the whole workgroup
+    const int row0 = p.chunk_rows ? p.chunk_rows[z] : 0;
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // uniform: descriptors depend on it
+    const int D = p.H * kDh;
+    const float* qkv = p.qkv + (size_t)row0 * p.ldq;
+    const TileSrc qs{qkv + h * kDh, p.ldq, T};
+    const TileSrc ks{qkv + D + h * kDh, p.ldq, T};
+    const TileSrc vs{qkv + 2 * D + h * kDh, p.ldq, T};
+    const TileSrc ps{p.P + (size_t)(p.T - T) * p.ldp + h * kDh, p.ldp, 2 * T - 1};
+
+    // The wave's blocks: n_a of keys, then n_b of positions.  Position block b
+    // starts at m = T - ROWS - r0 + 16 b; for row tile t it is block
+    // c = b - (RT-1-t) of the shifted band, where row 4 g + v's score of position
+    // j belongs to column 16 c + j + 4 g + v - 15.
+    const int blocks_a = (T + 15) / 16, blocks_b = (T + 30) / 16 + RT - 1;
+    const int n_a = max(0, (blocks_a - w + NW - 1) / NW), n_b = max(0, (blocks_b - w + NW - 1) / NW);
+    auto load = [&](auto& k, int n) {
+        if (n < n_a) {
+            k.load(ks.at(16 * (w + NW * n)), 0, p.ldq);
+        } else {
+            const int m0 = T - ROWS - r0 + 16 * (w + NW * (n - n_a));
+            k.load(ps.at(max(m0, 0)), min(m0, 0), p.ldp);
+        }
+    };
+    float* buf = smem + (RT + w) * kScoreRows;
+    ScoreRows in;
+    ScoreRow k0, k1;
+    if constexpr (kStage) {
+        load(in, 0);
+        if (w < RT) {
+            ScoreRows x;
+            x.load(qs.at(r0), 16 * w, p.ldq);
+            x.put(Q + w * kScoreRows);
+        }
+    } else {
+        load(k0, 0);
+        load(k1, 1);
+    }
+    // Q + bias (encoder.c:319-338); rows past T hold the bias alone and feed
+    // scores that nothing reads
+    ScoreRow q[RT];
+    auto load_q = [&](const float* bias) {
+        const auto rs = tiles::make_rsrc(bias + h * kDh, 4 * kDh);
+        v4f b[4][2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                b[i][x] = __builtin_bit_cast(v4f, tiles::ld_v4(rs, 4u * (32 * i + 8 * g + 4 * x)));
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            if constexpr (kStage) q[t].get(Q + t * kScoreRows);
+            else q[t].load(qs.at(r0), 16 * t, p.ldq);
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int l = 0; l < 8; ++l)
+                    q[t].v[i][l >> 2][l & 3] = __fadd_rn(q[t].at(i, l), b[i][l >> 2][l & 3]);
+        }
+    };
+    auto item = [&](int n, const ScoreRow& k) {
+        if (n == n_a) {                                     // every AC score is in place
+            load_q(p.pos_bias_v);
+            __syncthreads();
+        }
+        // o[t][v] = row 16 t + 4 g + v of q . row j of k
+        v4f acc[RT][8];
+        float o[RT][4];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int l = 0; l < 8; ++l) acc[t][l] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+                    acc[t][l] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[t].at(i, l), k.at(i, l), acc[t][l], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float s8[8];
+#pragma unroll
+                for (int l = 0; l < 8; ++l) s8[l] = acc[t][l][v];
+                o[t][v] = hsum8(s8);
+            }
+        if (n < n_a) {
+            const int col = 16 * (w + NW * n) + j;
+            if (col < T)
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) S[(16 * t + 4 * g + v) * sld + col] = o[t][v];
+            return;
+        }
+        // every (row, column) takes exactly one shifted value: read the scores
+        // first, then write them back combined
+        const int c0 = 16 * (w + NW * (n - n_a)) + j + 4 * g - 15;
+        float sc[RT][4];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = c0 - 16 * (RT - 1 - t) + v;
+                sc[t][v] = S[(unsigned)col < (unsigned)T ? (16 * t + 4 * g + v) * sld + col : 0];
+            }
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = c0 - 16 * (RT - 1 - t) + v;
+                if ((unsigned)col < (unsigned)T)
+                    S[(16 * t + 4 * g + v) * sld + col] = __fmul_rn(__fadd_rn(sc[t][v], o[t][v]), kScoreScale);
+            }
+    };
+    if constexpr (kStage) {
+        in.put(buf);
+        k0.get(buf);
+        load(in, 1);
+        __syncthreads();                                     // Q is in place
+        load_q(p.pos_bias_u);
+        for (int n = 0; n < n_a + n_b; n += 2) {
+            in.put(buf);
+            k1.get(buf);
+            load(in, n + 2);
+            item(n, k0);
+            if (n + 1 >= n_a + n_b) break;
+            in.put(buf);
+            k0.get(buf);
+            load(in, n + 3);
+            item(n + 1, k1);
+        }
+    } else {
+        load_q(p.pos_bias_u);
+        for (int n = 0; n < n_a + n_b; n += 2) {
+            item(n, k0);
+            load(k0, n + 2);
+            if (n + 1 >= n_a + n_b) break;
+            item(n + 1, k1);
+            load(k1, n + 3);
+        }
+    }
+    if (n_b == 0) __syncthreads();                           // the AC barrier of a wave without positions
+
+    // the first values, and those of the last T % 4 keys, during the softmax
+    const int col = 16 * CW * w + CW * j;                    // this lane's output columns
+    auto ld_cw = [&](__amdgpu_buffer_rsrc_t rs, int row) {
+        const int off = (int)(((uint32_t)row * (uint32_t)p.ldq + col) * 4u);
+        if constexpr (CW == 2) return __builtin_bit_cast(vcw, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+        else return __builtin_bit_cast(vcw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+    };
+    auto at_cw = [](const vcw& x, int c) { return __builtin_bit_cast(std::array<float, CW>, x)[c]; };
+    struct Values { vcw v[8]; };
+    auto load_v = [&](Values& x, int s) {                    // keys 32 s + 4 u + g
+        const auto rs = vs.at(32 * s);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x.v[u] = ld_cw(rs, 4 * u + g);
+    };
+    constexpr int VS = 4;
+    Values val[VS];
+#pragma unroll
+    for (int i = 0; i < VS; ++i) load_v(val[i], i);
+    const int T4 = T & ~3;
+    vcw vt[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) vt[u] = ld_cw(vs.at(T4), u);
+    __syncthreads();
+    for (int rl = 4 * w + g; rl < ROWS; rl += 4 * NW)
+        if (r0 + rl < T) softmax_row16(S + rl * sld, T);
+    __syncthreads();
+
+    // out[row][h*128 + d] = sum over keys ascending of S[row][key] * V[key][d]
+    v4f acc[RT][CW];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) acc[t][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    const float* srow = S + j * sld + g;
+    const int ng = T4 / 32, rest = (T4 & 31) / 4;
+    auto pv = [&](const Values& x, int s, auto full) {
+        float a[RT][8];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[t][u] = full || u < rest ? srow[16 * t * sld + 32 * s + 4 * u] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (full || u < rest)
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+#pragma unroll
+                    for (int c = 0; c < CW; ++c)
+                        acc[t][c] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][u], at_cw(x.v[u], c), acc[t][c], 0, 0, 0);
+    };
+    for (int s0 = 0; s0 <= ng; s0 += VS) {
+#pragma unroll
+        for (int i = 0; i < VS; ++i) {
+            if (s0 + i < ng) {
+                pv(val[i], s0 + i, std::true_type{});
+                load_v(val[i], s0 + i + VS);
+            } else if (s0 + i == ng && rest) {
+                pv(val[i], ng, std::false_type{});
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+        if (T4 + u < T)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float a = S[(16 * t + 4 * g + v) * sld + T4 + u];
+#pragma unroll
+                    for (int c = 0; c < CW; ++c) acc[t][c][v] = __fmaf_rn(a, at_cw(vt[u], c), acc[t][c][v]);
+                }
+    float* out = p.out + (size_t)row0 * p.ldo + h * kDh + col;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = r0 + 16 * t + 4 * g + v;
+            if (r < T)
+#pragma unroll
+                for (int c = 0; c < CW; ++c) out[(size_t)r * p.ldo + c] = acc[t][c][v];
+        }
+}
+
+// Sequences whose score rows do not fit in LDS beside rel_pos_attention4's
+// buffers (T > 1344): the block's score rows live in its own slice of p.scores
+// (task order); __syncthreads orders the workgroup's global writes as it does its
+// LDS writes.  32 rows share each key, position and value tile here, which
+// counts once the scores themselves go through memory: 284 us at T = 1400,
+// against 399 for rel_pos_attention4 with its scores there.
+__global__ __launch_bounds__(256, 2) void rel_pos_attention_long(AttnArgs p)
+{
+    extern __shared__ float tile[];                          // one staging tile
     const int sld = attn_sld(p.T);
 
     // (row block, head, chunk) in XCD runs
     int rb, h, z;
     const int task = attn_task(rb, h, z);
-    float* S = kGlobal ? p.scores + (size_t)task * kAttnRows * sld : smem;
-    float* tile = kGlobal ? smem : smem + kAttnRows * sld;
+    float* S = p.scores + (size_t)task * kAttnRows * sld;
     const int T = p.chunk_T ? p.chunk_T[z] : p.T;           // this chunk's rows
     const int r0 = rb * kAttnRows;
     if (r0 >= T) return;                                     // the whole workgroup
@@ -625,7 +1003,7 @@ __global__ __launch_bounds__(256, 2) void rel_pos_attention(AttnArgs p)
 // split as the split GEMM kernels split theirs (x = hi + lo + r, hi =
 // bf16(x), lo = bf16(x - hi), r below 2^-16 |x|): three products hi hi +
 // lo hi + hi lo per pair, within about 1e-5 of the exact kernel.  The
-// organisation is rel_pos_attention's: 32 query rows of one head of one
+// organisation is rel_pos_attention_long's: 32 query rows of one head of one
 // chunk per workgroup, their score rows in LDS, the content scores, then
 // the relative-position term added at the shifted positions, softmax, then
 // scores x V.  Fragments of v_mfma_f32_16x16x32_bf16: lane l = i + 16 g
@@ -646,7 +1024,7 @@ typedef __bf16 fa_v8bf __attribute__((ext_vector_type(8)));
 constexpr int kFragFloats = 512;                  // one fragment, hi and lo, 2 KB
 // Score-row stride of the split kernel, 4 more than a multiple of 32 floats:
 // the 4 lane groups of a result store, and the 16 rows of a fragment read,
-// start 4 or 16 banks apart (8 apart, rel_pos_attention's stride, put the
+// start 4 or 16 banks apart (8 apart, rel_pos_attention_long's stride, put the
 // 4 groups of a store on the same banks).
 __host__ __device__ constexpr int fa_sld(int T) { return ((T + 31) & ~31) + 4; }
 
@@ -1021,218 +1399,6 @@ __global__ __launch_bounds__(256, 2) void rel_pos_attention_fast(AttnArgs p, con
         }
 }
 
-// ---- short sequences (T <= kAttnShortT) -------------------------------------
-// A workgroup of 4 waves takes kAttnShortRows = 16 query rows, 4 per wave.
-// Every key, position and value row it reads is loaded into LDS at once,
-// behind one barrier: keys [0, 64), positions [m_first, m_first + 64 nb)
-// (nb 64-row blocks cover the block's shifted positions), values [0, T
-// rounded up to 16).  Rows past an operand's end read 0.  After the barrier
-// each wave runs its own rows without waiting for the others.  It performs
-// the operations of rel_pos_attention, each output through the same chain in
-// the same order, so the bits are the same:
-// - AC, and BD with the shift and the scale;
-// - the softmax;
-// - scores x V.
-// Only the work division differs: 4 rows a wave instead of 8, and one
-// staging round trip instead of one per 64-row tile.
-
-// acc[t % 8] += A(step t) * b[t] for the 16 steps of one A register.
-template <int... Ts>
-__device__ inline void score_steps1(std::integer_sequence<int, Ts...>, float a, const float (&b)[16],
-                                    v4f (&acc)[8])
-{
-    ((acc[Ts & 7] = mfma_bcast<Ts>(a, b[Ts], acc[Ts & 7])), ...);
-}
-
-// 4 rows x 64 columns of NT dot products over k = 0..127: a[kb] holds the 4
-// rows in broadcast layout for k in [16 kb, 16 kb + 16), lane j's B row is
-// brow (128 floats in LDS).  Chain t % 8 of each output takes k ascending;
-// the 8 chains are reduced as hsum8 (score_half and score_sums' order).
-__device__ inline void score_rows(const float* brow, const float (&a)[8], float (&out)[4])
-{
-    v4f acc[8];
-#pragma unroll
-    for (int l = 0; l < 8; ++l) acc[l] = v4f{0.f, 0.f, 0.f, 0.f};
-    float b[2][16];
-    auto fetch = [&](float (&dst)[16], int kb) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 v = *reinterpret_cast<const float4*>(brow + kb * 16 + 4 * q);
-            dst[4 * q] = v.x; dst[4 * q + 1] = v.y; dst[4 * q + 2] = v.z; dst[4 * q + 3] = v.w;
-        }
-    };
-    fetch(b[0], 0);
-#pragma unroll
-    for (int kb = 0; kb < 8; ++kb) {
-        if (kb + 1 < 8) fetch(b[(kb + 1) & 1], kb + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        score_steps1(std::make_integer_sequence<int, 16>{}, a[kb], b[kb & 1], acc);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float s8[8];
-#pragma unroll
-        for (int l = 0; l < 8; ++l) s8[l] = acc[l][i];
-        out[i] = hsum8(s8);
-    }
-}
-
-// scores x V for 4 rows: acc[d] += S[row i][j0 + t] * V[j0 + t][64 d + lane].
-template <int... Ts>
-__device__ inline void pv_steps1_full(std::integer_sequence<int, Ts...>, float a, const float* vt,
-                                      v4f (&acc)[2])
-{
-    const int lane = threadIdx.x & 63;
-    float b0[16], b1[16];
-    ((b0[Ts] = vt[Ts * kTileLd + lane], b1[Ts] = vt[Ts * kTileLd + 64 + lane]), ...);
-    ((acc[0] = mfma_bcast<Ts>(a, b0[Ts], acc[0]), acc[1] = mfma_bcast<Ts>(a, b1[Ts], acc[1])), ...);
-}
-
-template <int... Ts>
-__device__ inline void pv_steps1(std::integer_sequence<int, Ts...>, float a, const float* vt, int n,
-                                 v4f (&acc)[2])
-{
-    const int lane = threadIdx.x & 63;
-    (((Ts < n) ? (acc[0] = mfma_bcast<Ts>(a, vt[Ts * kTileLd + lane], acc[0]),
-                  acc[1] = mfma_bcast<Ts>(a, vt[Ts * kTileLd + 64 + lane], acc[1]), 0)
-               : 0), ...);
-}
-
-__global__ __launch_bounds__(256) void rel_pos_attention_short(AttnArgs p)
-{
-    // Score rows [kAttnShortRows][sld], then the staged rows [n_rows][kTileLd].
-    extern __shared__ float smem[];
-    const int sld = attn_sld(p.T);
-    int rb, h, z;
-    attn_task(rb, h, z);
-    const int T = p.chunk_T ? p.chunk_T[z] : p.T;           // this chunk's rows
-    const int r0 = rb * kAttnShortRows;
-    if (r0 >= T) return;                                     // the whole workgroup
-    const int row0 = p.chunk_rows ? p.chunk_rows[z] : 0;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int D = p.H * kDh;
-    const float* qkv = p.qkv + (size_t)row0 * p.ldq;
-    const float* K = qkv + D + h * kDh;
-    const float* V = qkv + 2 * D + h * kDh;
-    const float* P = p.P + (size_t)(p.T - T) * p.ldp + h * kDh;
-    const int r_hi = min(r0 + kAttnShortRows, T) - 1;
-    const int L = 2 * T - 1;
-    const int m_first = T - 1 - r_hi, m_last = 2 * T - 2 - r0;
-    const int nb = (m_last - m_first + 64) / 64;             // position blocks: 1 or 2
-    const int n_rows = 64 + 64 * nb + ((T + 15) & ~15);      // keys, positions, values
-    float* S = smem;
-    float* kt = smem + kAttnShortRows * sld;                 // staged row s at kt + s kTileLd
-    float* pt = kt + 64 * kTileLd;
-    float* vt = pt + 64 * nb * kTileLd;
-
-    // This wave's Q rows in broadcast layout (lane 4t + i: row r0 + 4w + i at
-    // k = 16 kb + t), loaded with the staged rows; rows past T read row T-1
-    // and are zeroed after.
-    const int i = lane & 3, t = lane >> 2;
-    const int rq = r0 + 4 * w + i;
-    float qv[8], bu[8], bv[8];
-    {
-        const float* q = qkv + (size_t)min(rq, T - 1) * p.ldq + h * kDh;
-#pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            qv[kb] = q[16 * kb + t];
-            bu[kb] = p.pos_bias_u[h * kDh + 16 * kb + t];
-            bv[kb] = p.pos_bias_v[h * kDh + 16 * kb + t];
-        }
-    }
-    // Staged row s (32 float4 per row, 8 rows per pass of the 256 threads):
-    // key s for s < 64, position m_first + s - 64 below 64 + 64 nb, then
-    // value s - 64 - 64 nb.  Region bounds are multiples of 16 rows, so each
-    // pass reads one region and its branch is uniform.
-    {
-        constexpr int kPass = (64 + 128 + kAttnShortT) / 8;
-        const TileSrc ks{K, p.ldq, T}, ps{P, p.ldp, L}, vs{V, p.ldq, T};
-        const __amdgpu_buffer_rsrc_t rk = ks.at(0), rp = ps.at(m_first), rv = vs.at(0);
-        const int sr = threadIdx.x >> 5, c = 4 * (threadIdx.x & 31);
-        float4 st[kPass];
-#pragma unroll
-        for (int q = 0; q < kPass; ++q) {
-            const int s0 = 8 * q, s = s0 + sr;
-            if (s0 < n_rows) {
-                tiles::v4u u;
-                if (s0 < 64)
-                    u = tiles::ld_v4(rk, (uint32_t)(s * p.ldq + c) * 4u);
-                else if (s0 < 64 + 64 * nb)
-                    u = tiles::ld_v4(rp, (uint32_t)((s - 64) * p.ldp + c) * 4u);
-                else
-                    u = tiles::ld_v4(rv, (uint32_t)((s - 64 - 64 * nb) * p.ldq + c) * 4u);
-                st[q] = as_float4(u);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < kPass; ++q)
-            if (8 * q < n_rows) *reinterpret_cast<float4*>(kt + (8 * q + sr) * kTileLd + c) = st[q];
-    }
-    float au[8], av[8];
-    {
-        const bool live = rq < T;
-#pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            au[kb] = live ? __fadd_rn(qv[kb], bu[kb]) : 0.0f;
-            av[kb] = live ? __fadd_rn(qv[kb], bv[kb]) : 0.0f;
-        }
-    }
-    __syncthreads();
-
-    // From here on a wave reads and writes only its own 4 score rows (LDS
-    // accesses of one wave complete in order): no more barriers.
-    float* Sw = S + 4 * w * sld;
-    {   // AC: S[row][j] = Q_u[row] . K[j], j = lane
-        float o[4];
-        score_rows(kt + lane * kTileLd, au, o);
-        if (lane < T)
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii) Sw[ii * sld + lane] = o[ii];
-    }
-    // BD at the shifted positions m = T-1-row+j, combined and scaled
-    for (int b = 0; b < nb; ++b) {
-        const int m0 = m_first + 64 * b;
-        float o[4];
-        score_rows(pt + (64 * b + lane) * kTileLd, av, o);
-        const int jb = m0 + lane - (T - 1) + r0;
-        float sc[4];
-        bool ok[4];
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) {
-            const int rl = 4 * w + ii;
-            ok[ii] = r0 + rl < T && (unsigned)(jb + rl) < (unsigned)T;
-            sc[ii] = S[ok[ii] ? jb + rl * (sld + 1) : 0];
-        }
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii)
-            if (ok[ii])
-                S[jb + (4 * w + ii) * (sld + 1)] = __fmul_rn(__fadd_rn(sc[ii], o[ii]), kScoreScale);
-    }
-    // softmax: lanes 0..31, 8 per row
-    if (lane < 32) softmax_row(Sw + (lane >> 3) * sld, T, r0 + 4 * w + (lane >> 3) < T);
-
-    // out[row][h*128 + d] = sum over j ascending of S[row][j] * V[j][d]
-    v4f acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-    const float* srow = Sw + i * sld + t;
-    int j0 = 0;
-    for (; j0 + 16 <= T; j0 += 16)
-        pv_steps1_full(std::make_integer_sequence<int, 16>{}, srow[j0], vt + j0 * kTileLd, acc);
-    if (T & 15) {
-        const float a = j0 + t < T ? srow[j0] : 0.0f;
-        pv_steps1(std::make_integer_sequence<int, 16>{}, a, vt + j0 * kTileLd, T & 15, acc);
-    }
-    float* out = p.out + (size_t)row0 * p.ldo + h * kDh;
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-        const int r = r0 + 4 * w + ii;
-        if (r < T) {
-            out[(size_t)r * p.ldo + lane] = acc[0][ii];
-            out[(size_t)r * p.ldo + 64 + lane] = acc[1][ii];
-        }
-    }
-}
-
 // ---- GLU (encoder.c:453-461) -------------------------------------------------
 // gated[r][d] = va * (1 / (1 + exp(-vb))), va = in[r][d], vb = in[r][D + d].
 __device__ inline float glu_value(float va, float vb)
@@ -1508,45 +1674,42 @@ hipError_t launch_layer_norm_split(const float* x, int ldx, const float* gamma, 
     return hipGetLastError();
 }
 
-// PK_GPU_ATTN_SHORT=0 sends short sequences to rel_pos_attention too (the
-// same bits; for comparing the two).
-bool attn_short_enabled()
-{
-    static const bool on = [] {
-        const char* v = getenv("PK_GPU_ATTN_SHORT");
-        return !(v && strcmp(v, "0") == 0);
-    }();
-    return on;
-}
-
+// Which attention kernel: by the workgroups that 16 and 32 query rows a
+// workgroup make of the launch (us, one sequence of 8 heads unless said):
+// - up to one 16-row workgroup a CU, its operands staged: 23.5 at T = 416, where
+//   32 rows, unstaged, take 39.4; also beyond T = 1024, where 32 rows' scores
+//   leave one workgroup a CU (142 against 158 at T = 1101);
+// - up to one 32-row workgroup a CU: 8 waves, unstaged: 58.5 at T = 700 (16 rows
+//   staged 66.2, 32 rows by 4 waves 63.2);
+// - more (an encoder's chunks): 4 waves, unstaged, two workgroups a CU: exact
+//   encoder at 3200 frames 37.6 ms (8 waves 38.4, 16 rows staged 38.2);
+// - scores that do not fit in LDS: rel_pos_attention_long.
 hipError_t launch_attention(const AttnArgs& a, int n_chunks, hipStream_t s)
 {
     if (a.T <= 0 || n_chunks <= 0) return hipSuccess;
-    dim3 grid((a.T + kAttnRows - 1) / kAttnRows, a.H, n_chunks);
-    if (a.T > kAttnMaxT) {
-        // score rows in the caller's workspace; LDS holds the staging tile only
-        if (!a.scores) return hipErrorInvalidValue;
+    if (a.T > kAttnMaxT && !a.scores) return hipErrorInvalidValue;      // attn_scores_floats asks for it
+    if (attn_lds_bytes(a.T, 1, 8, true) > kLdsBytes) {
+        const dim3 grid((a.T + kAttnRows - 1) / kAttnRows, a.H, n_chunks);
         if ((size_t)grid.x * grid.y * grid.z * kAttnRows * attn_sld(a.T) >= ((size_t)1 << 40))
             return hipErrorInvalidValue;
-        hipLaunchKernelGGL(rel_pos_attention<true>, grid, dim3(256), 4u * kTileFloats, s, a);
+        hipLaunchKernelGGL(rel_pos_attention_long, grid, dim3(256), 4u * kTileFloats, s, a);
         return hipGetLastError();
     }
-    if (a.T <= kAttnShortT && attn_short_enabled()) {
-        static const hipError_t attr_s = hipFuncSetAttribute(
-            reinterpret_cast<const void*>(&rel_pos_attention_short),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_short_lds_bytes(kAttnShortT));
-        if (attr_s != hipSuccess) return attr_s;
-        const dim3 gs((a.T + kAttnShortRows - 1) / kAttnShortRows, a.H, n_chunks);
-        hipLaunchKernelGGL(rel_pos_attention_short, gs, dim3(256), attn_short_lds_bytes(a.T), s, a);
+    auto run = [&](auto kern, int rt, int nw, bool stage) {
+        // LDS above the default dynamic limit is granted once per instantiation
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        if (attr != hipSuccess) return attr;
+        const dim3 grid((a.T + 16 * rt - 1) / (16 * rt), a.H, n_chunks);
+        hipLaunchKernelGGL(kern, grid, dim3(64 * nw), (unsigned)attn_lds_bytes(a.T, rt, nw, stage), s, a);
         return hipGetLastError();
-    }
-    // LDS above the default dynamic limit is granted once per process.
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&rel_pos_attention<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)attn_lds_bytes(kAttnMaxT));
-    if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(rel_pos_attention<false>, grid, dim3(256), attn_lds_bytes(a.T), s, a);
-    return hipGetLastError();
+    };
+    constexpr long long kCus = 256;
+    const long long n16 = (long long)((a.T + 15) / 16) * a.H * n_chunks;
+    const long long n32 = (long long)((a.T + 31) / 32) * a.H * n_chunks;
+    if (n16 <= kCus || a.T > 1024) return run(rel_pos_attention4<1, 8, true>, 1, 8, true);
+    if (n32 <= kCus) return run(rel_pos_attention4<2, 8, false>, 2, 8, false);
+    return run(rel_pos_attention4<2, 4, false>, 2, 4, false);
 }
 
 size_t attn_fast_ws_floats(int T, int H, int n_chunks)
