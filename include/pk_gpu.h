@@ -576,7 +576,7 @@ int pk_gpu_force_config(int index);
  * invalid), and a test hook that forces one for later GEMM calls on this
  * thread (-1 = automatic).  The tile never changes a result. */
 int pk_gpu_num_chain_tiles(void);
-int pk_gpu_pick_chain_tile(int M, int N, int bits);
+int pk_gpu_pick_chain_tile(int M, int N, int K, int bits);
 int pk_gpu_force_chain_tile(int tile);
 
 #ifdef __cplusplus

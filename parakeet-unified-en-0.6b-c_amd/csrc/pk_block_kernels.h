@@ -97,8 +97,9 @@ hipError_t launch_depthwise(const DwArgs& a, int n_chunks, hipStream_t s);
 hipError_t launch_transpose(const float* in, float* out, int R, int C, hipStream_t s);
 
 // Pre-encode subsampling (encoder.c:103-174), channel-last [H][W][256].
-hipError_t launch_conv0_relu(const float* mel, int T, int n_mels, const float* w, const float* b,
-                             float* out, int H1, int W1, hipStream_t s);
+hipError_t launch_conv0_conv2(const float* mel, int T, int n_mels, const float* w0, const float* b0,
+                              const float* w2, const float* b2, float* out, int H1, int W1, int H2, int W2,
+                              hipStream_t s);
 hipError_t launch_dwconv3x3s2(const float* in, int H, int W, const float* w, const float* b,
                               float* out, int Ho, int Wo, hipStream_t s);
 hipError_t launch_flatten_rows(const float* in, float* out, int H, int W, hipStream_t s);

@@ -1537,50 +1537,126 @@ __global__ __launch_bounds__(256) void depthwise_tiled(DwArgs p)
 
 constexpr int kSub = 256;          // PK_SUB_CHANNELS
 
-// conv.0: 1 -> 256 channels, 3x3, stride 2, pad 1, over the image whose row
-// t is mel frame t (mel [n_mels][T], encoder.c:110-120), then ReLU.  One
-// workgroup per output row oh and run of kC0Run output columns, one thread
-// per channel: the run's input window (3 frames x 2 kC0Run + 1 mel bins, 0
-// outside the image) is staged in LDS by one load per thread, a channel's
-// nine weights and bias are read once, and each position stores 256
-// consecutive floats.  pk_conv2d skips the taps outside the image; here they
-// take part with x = 0.  fma(0, w, v) is v except that a zero v may change
-// sign, and the ReLU maps either zero to +0, so the outputs are the same.
-constexpr int kC0Run = 16;
-constexpr int kC0Win = 2 * kC0Run + 1;
+// conv.0 (1 -> 256 channels, 3x3, stride 2, pad 1, over the image whose row t is
+// mel frame t; mel [n_mels][T], encoder.c:110-120) and its ReLU, then conv.2
+// (depthwise 3x3, stride 2, pad 1) of the result.  conv.0's output is the
+// largest array of the pre-encode (839 MB for 25600 frames, 178 us to write at
+// the chip's copy rate and as much to read back), so it stays in registers: a
+// thread is one channel and keeps three columns of 2 kFcRows + 1 conv.0 values, a
+// workgroup produces kFcRows x kFcCols outputs of conv.2.  Neighbouring rows of
+// workgroups both compute the conv.0 row between them (1/9 more work).  Every
+// output is the same chain as from memory.  Bound by its VALU instructions
+// (about 60 per output); 25600 frames: 555 us as two kernels, XXX as this one.
+//
+// The mel window (zeros outside the image) is staged in LDS by mel bin, so a bin's
+// frames are 16-byte reads that all lanes share.  pk_conv2d skips the taps outside
+// the image; here conv.0's take part with x = 0.  fma(0, w, v) is v except that a
+// zero v may change sign, and the ReLU maps either zero to +0, so the outputs are
+// the same.  conv.2's are skipped.
+constexpr int kFcRows = 4, kFcCols = 8;
 
-__global__ __launch_bounds__(kSub) void conv0_relu(const float* __restrict__ mel, int T, int n_mels,
-                                                   const float* __restrict__ w,
-                                                   const float* __restrict__ b, float* out, int H1,
-                                                   int W1)
+__global__ __launch_bounds__(kSub) void conv0_conv2(const float* __restrict__ mel, int T, int n_mels,
+                                                    const float* __restrict__ w0, const float* __restrict__ b0,
+                                                    const float* __restrict__ w2, const float* __restrict__ b2,
+                                                    float* out, int H1, int W1, int H2, int W2)
 {
-    __shared__ float win[3 * kC0Win];
+    constexpr int NR = 2 * kFcRows + 1;               // conv.0 rows of the block
+    constexpr int MR = 2 * NR + 2, MB = 4 * kFcCols + 3;      // mel frames (19 and a pad) and bins
+    static_assert(MR % 4 == 0, "16-byte rows");
+    __shared__ __attribute__((aligned(16))) float win[MB][MR];
     const int c = threadIdx.x;
-    const int oh = blockIdx.x, ow0 = blockIdx.y * kC0Run;
-    const int ih0 = 2 * oh - 1, iw0 = 2 * ow0 - 1;
-    if (c < 3 * kC0Win) {
-        const int ih = ih0 + c / kC0Win, iw = iw0 + c % kC0Win;
-        win[c] = ih >= 0 && ih < T && iw >= 0 && iw < n_mels ? mel[(size_t)iw * T + ih] : 0.0f;
+    const int oh0 = blockIdx.x * kFcRows, ow0 = blockIdx.y * kFcCols;
+    const int ih0 = 4 * oh0 - 3, ib0 = 4 * ow0 - 3;   // first mel frame and bin of the window
+    for (int i = c; i < MB * MR; i += kSub) {
+        const int ib = ib0 + i / MR, ih = ih0 + i % MR;
+        win[i / MR][i % MR] = ih >= 0 && ih < T && ib >= 0 && ib < n_mels ? mel[(size_t)ib * T + ih] : 0.0f;
     }
-    float wv[9];
+    float u[9], w[9];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) wv[k] = w[c * 9 + k];
-    const float bias = b[c];
+    for (int k = 0; k < 9; ++k) {
+        u[k] = w0[c * 9 + k];
+        w[k] = w2[c * 9 + k];
+    }
+    const float ub = b0[c], wb = b2[c];
     __syncthreads();
-    const int nr = min(kC0Run, W1 - ow0);
-    float* o = out + ((size_t)oh * W1 + ow0) * kSub + c;
+
+    float x[3][NR];                                   // conv.0 columns 2 ow - 1 .. 2 ow + 1
+    float m[3][MR];                                   // mel bins of one of them
+    auto bin = [&](float (&d)[MR], int b) {
 #pragma unroll
-    for (int r = 0; r < kC0Run; ++r) {
-        if (r < nr) {
-            float v = bias;
-#pragma unroll
-            for (int k = 0; k < 9; ++k) v = __fmaf_rn(win[(k / 3) * kC0Win + 2 * r + k % 3], wv[k], v);
-            o[(size_t)r * kSub] = v > 0.0f ? v : 0.0f;
+        for (int q = 0; q < MR; q += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(&win[b][q]);
+            d[q] = v.x; d[q + 1] = v.y; d[q + 2] = v.z; d[q + 3] = v.w;
         }
+    };
+    auto column = [&](float (&o)[NR], const float (&m0)[MR], const float (&m1)[MR], const float (&m2)[MR]) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            float v = ub;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                const float in = k % 3 == 0 ? m0[2 * r + k / 3] : k % 3 == 1 ? m1[2 * r + k / 3] : m2[2 * r + k / 3];
+                v = __fmaf_rn(in, u[k], v);
+            }
+            o[r] = v > 0.0f ? v : 0.0f;
+        }
+    };
+    // taps outside conv.0's image: the first row and column, and past the last
+    const bool inside = oh0 > 0 && 2 * oh0 - 1 + NR <= H1;
+    bin(m[0], 0);
+    bin(m[1], 1);
+    bin(m[2], 2);
+    column(x[0], m[0], m[1], m[2]);
+    const int nc = min(kFcCols, W2 - ow0), nr = min(kFcRows, H2 - oh0);
+    float* o = out + ((size_t)oh0 * W2 + ow0) * kSub + c;
+    // one output column: columns A, B, C of x are 2 ow - 1, 2 ow, 2 ow + 1
+    auto outputs = [&](int j, const float (&xa)[NR], const float (&xb)[NR], const float (&xc)[NR]) {
+        const bool left = ow0 + j > 0, right = 2 * (ow0 + j) + 1 < W1;
+        if (inside && left && right) {
+#pragma unroll
+            for (int r = 0; r < kFcRows; ++r) {
+                float v = wb;
+#pragma unroll
+                for (int k = 0; k < 9; ++k)
+                    v = __fmaf_rn(k % 3 == 0 ? xa[2 * r + k / 3] : k % 3 == 1 ? xb[2 * r + k / 3] : xc[2 * r + k / 3],
+                                  w[k], v);
+                if (r < nr) o[((size_t)r * W2 + j) * kSub] = v;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < kFcRows; ++r) {
+                float v = wb;
+#pragma unroll
+                for (int k = 0; k < 9; ++k) {
+                    const int oh = 2 * (oh0 + r) - 1 + k / 3;
+                    const bool ok = oh >= 0 && oh < H1 && (k % 3 != 0 || left) && (k % 3 != 2 || right);
+                    const float t = __fmaf_rn(
+                        k % 3 == 0 ? xa[2 * r + k / 3] : k % 3 == 1 ? xb[2 * r + k / 3] : xc[2 * r + k / 3], w[k], v);
+                    v = ok ? t : v;
+                }
+                if (r < nr) o[((size_t)r * W2 + j) * kSub] = v;
+            }
+        }
+    };
+    // columns 2 j + 1 and 2 j + 2 of the block from bins 4 j + 2 .. 4 j + 6
+    auto step = [&](int j, float (&xa)[NR], float (&xb)[NR], float (&xc)[NR]) {
+        bin(m[0], 4 * j + 2);
+        bin(m[1], 4 * j + 3);
+        bin(m[2], 4 * j + 4);
+        column(xb, m[0], m[1], m[2]);
+        bin(m[0], 4 * j + 5);
+        bin(m[1], 4 * j + 6);
+        column(xc, m[2], m[0], m[1]);
+        outputs(j, xa, xb, xc);
+    };
+    for (int j = 0; j < nc; j += 2) {
+        step(j, x[0], x[1], x[2]);
+        if (j + 1 >= nc) break;
+        step(j + 1, x[2], x[1], x[0]);
     }
 }
 
-// Depthwise 3x3, stride 2, pad 1 (conv.2 and conv.5, groups = 256).
+// Depthwise 3x3, stride 2, pad 1 (conv.5, groups = 256).
 __global__ void dwconv3x3s2(const float* __restrict__ in, int H, int W,
                             const float* __restrict__ w, const float* __restrict__ b, float* out,
                             int Ho, int Wo)
@@ -1605,18 +1681,20 @@ __global__ void dwconv3x3s2(const float* __restrict__ in, int H, int W,
     out[idx] = v;
 }
 
-// rows x n of C set to bias[0..n): the starting value of a chain that the
-// reference begins at the bias.
-
 // [H][W][256] -> [H][256*W], element (c, w) of row h at c*W + w
 // (encoder.c:152-158).
-__global__ void flatten_rows(const float* __restrict__ in, float* out, int H, int W)
+__global__ __launch_bounds__(256) void flatten_rows(const float* __restrict__ in, float* out, int H, int W)
 {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int F = kSub * W;
-    if (idx >= (long long)H * F) return;
-    const int h = (int)(idx / F), r = (int)(idx % F), c = r / W, w = r % W;
-    out[idx] = in[((size_t)h * W + w) * kSub + c];
+    // a row of up to 16 columns turned in LDS: reads and writes are whole lines
+    __shared__ float t[16 * (kSub + 1)];
+    const int h = blockIdx.x, w0 = blockIdx.y * 16, nw = min(16, W - w0);
+    for (int i = threadIdx.x; i < nw * kSub; i += 256)
+        t[i / kSub * (kSub + 1) + i % kSub] = in[((size_t)h * W + w0) * kSub + i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < nw * kSub; i += 256) {
+        const int c = i / nw, w = i % nw;
+        out[(size_t)h * kSub * W + (size_t)c * W + w0 + w] = t[w * (kSub + 1) + c];
+    }
 }
 
 // x *= s in place (s = sqrtf(d_model) = 32, encoder.c:578-592: exact).
@@ -1790,12 +1868,13 @@ hipError_t launch_transpose(const float* in, float* out, int R, int C, hipStream
 
 static unsigned blocks_of(long long n) { return (unsigned)((n + 255) / 256); }
 
-hipError_t launch_conv0_relu(const float* mel, int T, int n_mels, const float* w, const float* b,
-                             float* out, int H1, int W1, hipStream_t s)
+hipError_t launch_conv0_conv2(const float* mel, int T, int n_mels, const float* w0, const float* b0,
+                              const float* w2, const float* b2, float* out, int H1, int W1, int H2, int W2,
+                              hipStream_t s)
 {
-    if (H1 <= 0 || W1 <= 0) return hipSuccess;
-    hipLaunchKernelGGL(conv0_relu, dim3(H1, (W1 + kC0Run - 1) / kC0Run), dim3(kSub), 0, s, mel, T,
-                       n_mels, w, b, out, H1, W1);
+    if (H2 <= 0 || W2 <= 0) return hipSuccess;
+    hipLaunchKernelGGL(conv0_conv2, dim3((H2 + kFcRows - 1) / kFcRows, (W2 + kFcCols - 1) / kFcCols), dim3(kSub), 0,
+                       s, mel, T, n_mels, w0, b0, w2, b2, out, H1, W1, H2, W2);
     return hipGetLastError();
 }
 
@@ -1810,9 +1889,8 @@ hipError_t launch_dwconv3x3s2(const float* in, int H, int W, const float* w, con
 
 hipError_t launch_flatten_rows(const float* in, float* out, int H, int W, hipStream_t s)
 {
-    const long long n = (long long)H * W * kSub;
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(flatten_rows, dim3(blocks_of(n)), dim3(256), 0, s, in, out, H, W);
+    if (H <= 0 || W <= 0) return hipSuccess;
+    hipLaunchKernelGGL(flatten_rows, dim3(H, (W + 15) / 16), dim3(256), 0, s, in, out, H, W);
     return hipGetLastError();
 }
 

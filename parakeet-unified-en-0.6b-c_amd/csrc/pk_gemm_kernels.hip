@@ -104,31 +104,42 @@ static int choose_index(int M, int N, int K, WeightKind kind = W_I8)
 int choose_config_index(int M, int N, int K, WeightKind kind) { return choose_index(M, N, K, kind); }
 
 namespace {
-// us for the first round of workgroups (one on every CU) and for each further
-// one at K = 1024, by weight format and tile (pk_chain4.h).  Fitted to all
-// tiles at M = 1..3312 over N = 1024..4096 and K = 1024, 4096 on MI355X; K
-// scales all of a row alike.  A CU's workgroups share its matrix cores, so a
-// further round costs its MFMAs, and the first one also the time that one
-// workgroup alone leaves them idle.  The 16 x 32 tile is the fastest until a
-// second round, 128 x 64 from about 20 outputs per thread of the chip on.
-struct Rounds { float first, next; };
+// The time a four-deep GEMM takes, by weight format and tile (pk_chain4.h), us:
+// its first round of workgroups (one on every CU) a + b k, every further one e + c
+// k, k = K / 1024, but no less than its operands take through the L2s, every row
+// tile reading all of W and every column tile all of A.  A CU's workgroups share
+// its matrix cores, so a further round costs its multiplies (c), and the first
+// one also the time that one workgroup alone leaves the cores idle (b).  Fitted
+// on MI355X to all tiles at M = 16..3312, N = 1024..4096, K = 1024 and 4096; the
+// pick takes 1 % more than the best tile on average there.  L2: 32 x 32 tiles of
+// 2000 x 1024 x 4096 fp32 (2.1 GB of operands) take 183 us instead of the 133 of
+// their rounds, 64 x 64 ones 131.
+struct Rounds { float a, b, e, c; };
 constexpr Rounds kChain4Rounds[3][chain4::kNumTiles] = {
-    /* fp32 */ {{6.5f, 3.8f}, {7.0f, 4.1f}, {10.3f, 7.4f}, {11.2f, 7.9f}, {18.6f, 16.2f}, {35.2f, 31.0f}},
-    /* int8 */ {{6.8f, 4.0f}, {9.5f, 4.6f}, {11.3f, 8.0f}, {13.8f, 9.0f}, {24.3f, 15.7f}, {40.6f, 32.0f}},
-    /* int4 */ {{6.7f, 4.5f}, {9.2f, 4.7f}, {10.7f, 7.6f}, {13.4f, 8.9f}, {22.9f, 16.8f}, {38.7f, 32.5f}},
+    /* fp32 */ {{2.9f, 3.9f, 0.1f, 3.75f}, {2.8f, 4.3f, 0.2f, 4.0f}, {3.2f, 7.3f, 0.5f, 6.9f},
+                {3.7f, 7.7f, 0.9f, 7.1f}, {4.8f, 14.8f, 1.7f, 14.0f}, {6.3f, 29.9f, 4.0f, 27.6f}},
+    /* int8 */ {{2.9f, 3.9f, 0.3f, 3.9f}, {3.2f, 5.9f, 0.3f, 4.4f}, {3.0f, 8.0f, 0.6f, 7.2f},
+                {4.0f, 9.2f, 1.2f, 7.7f}, {5.0f, 17.0f, 1.5f, 14.7f}, {6.2f, 31.8f, 3.0f, 29.0f}},
+    /* int4 */ {{2.9f, 3.8f, 0.5f, 4.0f}, {3.2f, 6.0f, 0.2f, 4.5f}, {2.5f, 8.2f, 0.4f, 7.2f},
+                {3.3f, 9.8f, 1.1f, 7.8f}, {4.7f, 17.6f, 2.3f, 14.5f}, {5.7f, 32.3f, 4.0f, 28.5f}},
 };
 constexpr int kCus = 256;
+constexpr double kL2BytesPerUs = 12e6;
 thread_local int t_chain_tile = -1;
 
-int chain4_pick(int M, int N, WeightKind kind)
+int chain4_pick(int M, int N, int K, WeightKind kind)
 {
+    const double k = K / 1024.0;
+    const double w_bytes = (kind == W_F32 ? 4.0 : kind == W_I8 ? 1.0 : 0.625) * K * N;
     int best = 0;
     double best_t = 0.0;
     for (int i = 0; i < chain4::kNumTiles; ++i) {
         const chain4::Chain4Tile& t = chain4::kTiles[i];
-        const long long wgs = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const long long rows = (M + t.bm - 1) / t.bm, cols = (N + t.bn - 1) / t.bn;
         const Rounds& r = kChain4Rounds[kind][i];
-        const double time = r.first + r.next * (double)((wgs + kCus - 1) / kCus - 1);
+        const double rounds = (double)((rows * cols + kCus - 1) / kCus);
+        const double compute = r.a + r.b * k + (rounds - 1) * (r.e + r.c * k);
+        const double time = std::max(compute, (rows * w_bytes + cols * 4.0 * M * K) / kL2BytesPerUs);
         if (i == 0 || time < best_t) {
             best = i;
             best_t = time;
@@ -238,7 +249,7 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, 
         // The four-deep chains: the same bits, faster at every size measured.
         // They read whole vectors and take A as it is; other operands stay on
         // the K = 1 tiles.
-        const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.kind);
+        const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.K, p.kind);
         switch (p.kind) {
         case W_F32: err = chain4::launch_f32(tile, a, stream); break;
         case W_I8:  err = chain4::launch_i8(tile, a, stream); break;
@@ -336,13 +347,13 @@ extern "C" {
 
 int pk_gpu_num_chain_tiles(void) { return pkgpu::chain4::kNumTiles; }
 
-int pk_gpu_pick_chain_tile(int M, int N, int bits)
+int pk_gpu_pick_chain_tile(int M, int N, int K, int bits)
 {
-    if (M <= 0 || N <= 0) return -1;
+    if (M <= 0 || N <= 0 || K <= 0) return -1;
     switch (bits) {
-    case 4: return pkgpu::chain4_pick(M, N, pkgpu::W_I4);
-    case 8: return pkgpu::chain4_pick(M, N, pkgpu::W_I8);
-    case 32: return pkgpu::chain4_pick(M, N, pkgpu::W_F32);
+    case 4: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I4);
+    case 8: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I8);
+    case 32: return pkgpu::chain4_pick(M, N, K, pkgpu::W_F32);
     default: return -1;
     }
 }

@@ -1189,14 +1189,14 @@ int pre_encode_queued(pk_gpu_encoder* e, const float* mel, int T, float* x, hipS
     const int H1 = half_up(T), W1 = half_up(kMels);
     const int H2 = half_up(H1), W2 = half_up(W1);
     const int H3 = half_up(H2), W3 = half_up(W2);
-    int rc = grow(&e->pre_a, &e->pre_a_n, (size_t)H1 * W1 * kSub, s);
+    int rc = grow(&e->pre_a, &e->pre_a_n, (size_t)H2 * W2 * kSub, s);
     if (!rc) rc = grow(&e->pre_b, &e->pre_b_n, (size_t)H2 * W2 * kSub, s);
     if (rc) return rc;
     float *A = e->pre_a, *B = e->pre_b;
-    // conv.0 + ReLU -> A [H1][W1][256]
-    if ((rc = check(pkgpu::launch_conv0_relu(mel, T, kMels, w.w0, w.b0, A, H1, W1, s), "conv.0"))) return rc;
-    // conv.2 (depthwise) -> B; conv.3 (pointwise) + ReLU -> A
-    if ((rc = check(pkgpu::launch_dwconv3x3s2(A, H1, W1, w.w2, w.b2, B, H2, W2, s), "conv.2"))) return rc;
+    // conv.0 + ReLU and conv.2 (depthwise) -> B; conv.3 (pointwise) + ReLU -> A
+    if ((rc = check(pkgpu::launch_conv0_conv2(mel, T, kMels, w.w0, w.b0, w.w2, w.b2, B, H1, W1, H2, W2, s),
+                    "conv.0 and conv.2")))
+        return rc;
     // Rows are independent, so long inputs run in slabs whose operands stay
     // under the chain kernels' 2 GiB extent.
     auto pointwise = [&](const DevWeight& wt, const float* bias, const float* in, float* out, int rows) {

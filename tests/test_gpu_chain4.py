@@ -139,12 +139,13 @@ def test_chain_tile_choice():
     for bits in BITS.values():
         for N in (1, 16, 256, 1024, 2048, 3072, 4096):
             for M in list(range(1, 700, 7)) + [1000, 1656, 2000, 3312, 5000, 204800]:
-                t = lib.pk_gpu_pick_chain_tile(M, N, bits)
-                assert t in TILES
-                taken.add(t)
-        assert lib.pk_gpu_pick_chain_tile(16, 1024, bits) == 0
-        assert lib.pk_gpu_pick_chain_tile(204800, 256, bits) >= 4
+                for K in (256, 1024, 4096):
+                    t = lib.pk_gpu_pick_chain_tile(M, N, K, bits)
+                    assert t in TILES
+                    taken.add(t)
+        assert lib.pk_gpu_pick_chain_tile(16, 1024, 1024, bits) == 0
+        assert lib.pk_gpu_pick_chain_tile(3312, 4096, 1024, bits) >= 4
     assert taken == set(TILES)
-    assert lib.pk_gpu_pick_chain_tile(16, 16, 7) == -1 and lib.pk_gpu_pick_chain_tile(0, 16, 8) == -1
+    assert lib.pk_gpu_pick_chain_tile(16, 16, 16, 7) == -1 and lib.pk_gpu_pick_chain_tile(0, 16, 16, 8) == -1
     assert lib.pk_gpu_force_chain_tile(len(TILES)) == -1
     assert lib.pk_gpu_force_chain_tile(-1) == 0
