@@ -38,6 +38,9 @@ struct GemmProblem {
     float* C; int ldc;
     const float* bias = nullptr;     // length N, or null
     Epilogue epi = EPI_NONE;         // the residual epilogues require beta == 0
+    // Other kernels run on the chip at the same time (a hint: it may change the
+    // tile of an exact GEMM, never a result).
+    bool shares_chip = false;
     // Chains start from chain_bias[j] instead of beta*C (beta must be 0 and
     // bias null): a convolution whose sum starts from its bias (pk_conv2d).
     const float* chain_bias = nullptr;

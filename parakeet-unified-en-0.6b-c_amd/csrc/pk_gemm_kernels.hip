@@ -114,6 +114,11 @@ namespace {
 // pick takes 1 % more than the best tile on average there.  L2: 32 x 32 tiles of
 // 2000 x 1024 x 4096 fp32 (2.1 GB of operands) take 183 us instead of the 133 of
 // their rounds, 64 x 64 ones 131.
+//
+// shares_chip: other kernels run beside the GEMM and take what its last round
+// leaves free, so a part of a round counts as that part; and 128 x 64 tiles, one
+// workgroup of whose registers fill a CU, are left out.  3200 frames in two row
+// groups: 38.2 ms with each GEMM's own best tile, 37.1 so (37.9 with 128 x 64).
 struct Rounds { float a, b, e, c; };
 constexpr Rounds kChain4Rounds[3][chain4::kNumTiles] = {
     /* fp32 */ {{2.9f, 3.9f, 0.1f, 3.75f}, {2.8f, 4.3f, 0.2f, 4.0f}, {3.2f, 7.3f, 0.5f, 6.9f},
@@ -127,17 +132,19 @@ constexpr int kCus = 256;
 constexpr double kL2BytesPerUs = 12e6;
 thread_local int t_chain_tile = -1;
 
-int chain4_pick(int M, int N, int K, WeightKind kind)
+int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip = false)
 {
     const double k = K / 1024.0;
     const double w_bytes = (kind == W_F32 ? 4.0 : kind == W_I8 ? 1.0 : 0.625) * K * N;
     int best = 0;
     double best_t = 0.0;
-    for (int i = 0; i < chain4::kNumTiles; ++i) {
+    const int n = chain4::kNumTiles - (shares_chip ? 1 : 0);
+    for (int i = 0; i < n; ++i) {
         const chain4::Chain4Tile& t = chain4::kTiles[i];
         const long long rows = (M + t.bm - 1) / t.bm, cols = (N + t.bn - 1) / t.bn;
         const Rounds& r = kChain4Rounds[kind][i];
-        const double rounds = (double)((rows * cols + kCus - 1) / kCus);
+        double rounds = (double)((rows * cols + kCus - 1) / kCus);
+        if (shares_chip) rounds = std::max(1.0, (double)(rows * cols) / kCus);
         const double compute = r.a + r.b * k + (rounds - 1) * (r.e + r.c * k);
         const double time = std::max(compute, (rows * w_bytes + cols * 4.0 * M * K) / kL2BytesPerUs);
         if (i == 0 || time < best_t) {
@@ -249,7 +256,7 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, 
         // The four-deep chains: the same bits, faster at every size measured.
         // They read whole vectors and take A as it is; other operands stay on
         // the K = 1 tiles.
-        const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.K, p.kind);
+        const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.K, p.kind, p.shares_chip);
         switch (p.kind) {
         case W_F32: err = chain4::launch_f32(tile, a, stream); break;
         case W_I8:  err = chain4::launch_i8(tile, a, stream); break;

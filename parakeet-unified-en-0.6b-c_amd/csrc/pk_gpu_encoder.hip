@@ -138,6 +138,7 @@ struct pk_gpu_encoder {
     // Row groups replayed concurrently: group 0 on the caller's stream, group
     // g > 0 on side[g - 1], joined through events around the replay.
     int n_groups = 2;
+    bool several_groups = false;        // the current run's row groups are more than one
     int lag = -1;                  // pk_gpu_encoder_set_group_lag (-1: group_lag())
     // fast numerics: LayerNorms feeding a GEMM write pre-split output
     // (PK_GPU_PRESPLIT=0 at creation turns it off; the results are the same)
@@ -403,11 +404,10 @@ GemmProblem block_problem(const DevWeight& w, const float* A, int M, float* C, c
     return p;
 }
 
-int gemm_launch(const DevWeight& w, const float* A, int M, float* C, const float* bias,
-                Epilogue epi, hipStream_t s, pkgpu::Tolerance tol = pkgpu::TOL_NONE,
-                float* work = nullptr, bool presplit = false, const FusedLn& ln = FusedLn())
+int gemm_launch(const DevWeight& w, const float* A, int M, float* C, const float* bias, Epilogue epi, hipStream_t s)
 {
-    return pkgpu::rt::gemm(block_problem(w, A, M, C, bias, epi, tol, work, presplit, ln), s, tol);
+    return pkgpu::rt::gemm(block_problem(w, A, M, C, bias, epi, pkgpu::TOL_NONE, nullptr, false, FusedLn()), s,
+                           pkgpu::TOL_NONE);
 }
 
 int check(hipError_t r, const char* what) { return r == hipSuccess ? PK_GPU_OK : hip_error(r, what); }
@@ -541,7 +541,9 @@ int gemm(pk_gpu_encoder* e, const DevWeight& w, const float* A, int M, float* C,
     const pkgpu::Tolerance tol = exact ? pkgpu::TOL_NONE : pkgpu::rt::tolerance_of(e->numerics);
     return timed(e, stage_of(w), flops, bytes, s,
                  [&] {
-                     return gemm_launch(w, A, M, C, bias, epi, s, tol, work, presplit, ln);
+                     GemmProblem p = block_problem(w, A, M, C, bias, epi, tol, work, presplit, ln);
+                     p.shares_chip = e->several_groups;
+                     return pkgpu::rt::gemm(p, s, tol);
                  });
 }
 
@@ -954,6 +956,7 @@ int run_queued(pk_gpu_encoder* e, const float* x, int T, int chunk, int ov, floa
     // length, with rows relative to the group; the lengths follow at entry
     // rows_cap.
     std::vector<RowGroup> groups = plan_groups(chunks, e->n_groups);
+    e->several_groups = groups.size() > 1;
     std::vector<int> table, lens;
     {
         size_t ci = 0;
