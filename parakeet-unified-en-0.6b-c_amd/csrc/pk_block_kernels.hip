@@ -1406,12 +1406,27 @@ __device__ inline float glu_value(float va, float vb)
     return __fmul_rn(va, __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_ieee(-vb))));
 }
 
-__global__ void glu_rows(const float* __restrict__ in, int ldi, float* out, int ldo, int rows, int D)
+// V consecutive elements a thread, counted in I: the division that finds the row is
+// a few instructions in 32 bits and most of the kernel in 64, where one element a
+// thread was bound by it (3200 x 1024, traced: 11.3 us, against 8.3 for its 39 MB
+// at the chip's copy rate).
+template <int V, typename I>
+__global__ __launch_bounds__(256) void glu_rows(const float* __restrict__ in, int ldi, float* out, int ldo, I units,
+                                                int D)
 {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)rows * D) return;
-    const int r = (int)(idx / D), d = (int)(idx % D);
-    out[(size_t)r * ldo + d] = glu_value(in[(size_t)r * ldi + d], in[(size_t)r * ldi + D + d]);
+    const I i = (I)blockIdx.x * 256 + threadIdx.x, per_row = (I)(D / V);
+    if (i >= units) return;
+    const I r = i / per_row;
+    const int d = (int)(i - r * per_row) * V;
+    const float* x = in + (size_t)r * ldi + d;
+    float* o = out + (size_t)r * ldo + d;
+    if constexpr (V == 4) {
+        const float4 u = *reinterpret_cast<const float4*>(x), v = *reinterpret_cast<const float4*>(x + D);
+        *reinterpret_cast<float4*>(o) =
+            make_float4(glu_value(u.x, v.x), glu_value(u.y, v.y), glu_value(u.z, v.z), glu_value(u.w, v.w));
+    } else {
+        *o = glu_value(x[0], x[D]);
+    }
 }
 
 // ---- depthwise convolution + Swish (tensor_ops.c:476-548, encoder.c:467-469)
@@ -1493,7 +1508,8 @@ __global__ __launch_bounds__(256) void depthwise_tiled(DwArgs p)
     constexpr int pad = (KK - 1) / 2, W = TB + KK - 1, WQ = (W + 3) / 4;
     __shared__ float win_s[W][64];
     const int z = blockIdx.z;
-    const int T = p.chunk_T ? p.chunk_T[z] : p.T;            // this chunk's rows
+    // this chunk's rows, uniform (see rel_pos_attention4)
+    const int T = __builtin_amdgcn_readfirstlane(p.chunk_T ? p.chunk_T[z] : p.T);
     const int t0 = blockIdx.x * TB;
     if (t0 >= T) return;                                     // the whole workgroup
     const int row0 = p.chunk_rows ? p.chunk_rows[z] : 0;
@@ -1508,6 +1524,10 @@ __global__ __launch_bounds__(256) void depthwise_tiled(DwArgs p)
         va[q] = x[(size_t)u * p.ldx];
         vb[q] = p.glu ? x[(size_t)u * p.ldx + p.C] : 0.0f;
     }
+    float wc[KK];                                            // in flight with the rows
+#pragma unroll
+    for (int k = 0; k < KK; ++k) wc[k] = p.w[(size_t)cc * KK + k];
+    const float bias = p.b ? p.b[cc] : 0.0f;
 #pragma unroll
     for (int q = 0; q < WQ; ++q) {
         const int j = slot + 4 * q, u = t0 - pad + j;
@@ -1515,10 +1535,6 @@ __global__ __launch_bounds__(256) void depthwise_tiled(DwArgs p)
     }
     __syncthreads();
     if (c >= p.C) return;
-    float wc[KK];
-#pragma unroll
-    for (int k = 0; k < KK; ++k) wc[k] = p.w[(size_t)c * KK + k];
-    const float bias = p.b ? p.b[c] : 0.0f;
 #pragma unroll
     for (int q = 0; q < TB / 4; ++q) {
         const int t = t0 + slot + 4 * q;
@@ -1546,7 +1562,7 @@ constexpr int kSub = 256;          // PK_SUB_CHANNELS
 // workgroup produces kFcRows x kFcCols outputs of conv.2.  Neighbouring rows of
 // workgroups both compute the conv.0 row between them (1/9 more work).  Every
 // output is the same chain as from memory.  Bound by its VALU instructions
-// (about 60 per output); 25600 frames: 555 us as two kernels, XXX as this one.
+// (about 60 per output); 25600 frames: 555 us as two kernels, about 90 as this one.
 //
 // The mel window (zeros outside the image) is staged in LDS by mel bin, so a bin's
 // frames are 16-byte reads that all lanes share.  pk_conv2d skips the taps outside
@@ -1835,8 +1851,21 @@ hipError_t launch_glu(const float* in, int ldi, float* out, int ldo, int rows, i
 {
     const long long n = (long long)rows * D;
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(glu_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, ldi, out,
-                       ldo, rows, D);
+    // 16-byte loads and stores where every row allows them; the last workgroup's
+    // numbers must fit in 32 bits too
+    const bool vec = D % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 &&
+                     (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+    const long long units = vec ? n / 4 : n;
+    const bool small = units < 0xffffff00LL;
+    const dim3 grid((unsigned)((units + 255) / 256));
+    if (vec && small)
+        hipLaunchKernelGGL((glu_rows<4, uint32_t>), grid, dim3(256), 0, s, in, ldi, out, ldo, (uint32_t)units, D);
+    else if (small)
+        hipLaunchKernelGGL((glu_rows<1, uint32_t>), grid, dim3(256), 0, s, in, ldi, out, ldo, (uint32_t)units, D);
+    else if (vec)
+        hipLaunchKernelGGL((glu_rows<4, uint64_t>), grid, dim3(256), 0, s, in, ldi, out, ldo, (uint64_t)units, D);
+    else
+        hipLaunchKernelGGL((glu_rows<1, uint64_t>), grid, dim3(256), 0, s, in, ldi, out, ldo, (uint64_t)units, D);
     return hipGetLastError();
 }
 
