@@ -310,7 +310,7 @@ def gemm_mode(specs, steps, warmup, min_weight_bytes=512 << 20, eager=False, for
                                         lib.pk_gpu_split_k_segments(m, n, k, bits) if split else None,
                           "config": None if small_m or split else
                                     (force_config if force_config >= 0 else
-                                     lib.pk_gpu_pick_config_bits(m, n, k, bits)),
+                                     f"four-deep tile {lib.pk_gpu_pick_chain_tile(m, n, k, bits)}"),
                           "avg_us": round(us, 2), "timing": "eager loop" if eager else "graph replay",
                           "tflops": round(tf, 2), "gbps": round(gbs, 1),
                           "frac_mfma_fp32": round(tf / PEAK_FP32_MFMA_TFLOPS, 4),
@@ -437,8 +437,8 @@ def ffn_mode(args):
     gbytes = (int4_bytes(D, FF) + int4_bytes(FF, D)) / gemm_s / 1e9
     frames_per_s = M * K / (elapsed_ms / 1e3)
 
-    cfg_up = lib.pk_gpu_pick_config_bits(M, FF, D, 4)
-    cfg_dn = lib.pk_gpu_pick_config_bits(M, D, FF, 4)
+    cfg_up = lib.pk_gpu_pick_chain_tile(M, FF, D, 4)
+    cfg_dn = lib.pk_gpu_pick_chain_tile(M, D, FF, 4)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "int4_ffn_pair_m375_traffic.json")
     if os.path.exists(tpath):
@@ -1127,10 +1127,9 @@ def encoder_mode(args):
         "roofline": {"bound": "mfma",
                      "kernel": "int4 feed-forward chain GEMM of the replay, M = "
                                f"{'/'.join(str(r) for r in group_rows)} per launch "
-                               "(1024->4096 with fused bias + Swish, tile config "
-                               f"{lib.pk_gpu_pick_config_bits(max(group_rows), FF, D, 4)}; "
-                               "4096->1024 with bias + half residual, tile config "
-                               f"{lib.pk_gpu_pick_config_bits(max(group_rows), D, FF, 4)})",
+                               "(1024->4096 with fused bias + Swish; 4096->1024 with bias + half "
+                               "residual; four-deep fp32 MFMA tiles chosen for row groups that "
+                               "share the chip)",
                      "achieved": round(i4_tflops, 2), "peak": PEAK_FP32_MFMA_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(i4_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
                      "traffic": traffic, "launches_per_step": i4_launches // KP,

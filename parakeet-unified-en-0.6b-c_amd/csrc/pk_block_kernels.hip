@@ -1562,7 +1562,7 @@ constexpr int kSub = 256;          // PK_SUB_CHANNELS
 // workgroup produces kFcRows x kFcCols outputs of conv.2.  Neighbouring rows of
 // workgroups both compute the conv.0 row between them (1/9 more work).  Every
 // output is the same chain as from memory.  Bound by its VALU instructions
-// (about 60 per output); 25600 frames: 555 us as two kernels, about 90 as this one.
+// (about 60 per output); 25600 frames: 555 us as two kernels, 92 as this one.
 //
 // The mel window (zeros outside the image) is staged in LDS by mel bin, so a bin's
 // frames are 16-byte reads that all lanes share.  pk_conv2d skips the taps outside

@@ -19,7 +19,7 @@
 // run in the producers.  What bounds the GEMMs after that: the producers'
 // VALU time (int4: 24 instructions per 8 weights), the last round of
 // workgroups, and the start and end of a launch.  Against the K = 1 tiles
-// (time in us, one box, hot weights):
+// (time in us on one MI355X, hot weights):
 //   int4   375 x 4096 x 1024   38.3 -> 30.9     375 x 1024 x 4096   51.1 -> 35.0
 //   int4  1656 x 4096 x 1024  163.4 -> 124.0   1656 x 1024 x 4096  144.5 -> 132.2
 //   int8  1656 x 3072 x 1024  109.2 -> 89.9     375 x 3072 x 1024   35.2 -> 28.4

@@ -1,4 +1,7 @@
-// pk_gemm_tiles.h - CDNA4 (gfx950) tile kernels of the quantized weight GEMMs.
+// pk_gemm_tiles.h - CDNA4 (gfx950) tile kernels of the quantized weight GEMMs on
+// the K = 1 fp32 MFMA forms.  They run the forced configurations and what the
+// four-deep tiles (pk_chain4.h) do not take: alpha other than 1, and operands
+// whose rows allow no vector loads.
 //
 // Numerics.  The reference computes every output as a sequential fused
 // multiply-add chain over k ascending, c = fma(fl(alpha*A[i][k]), w[k][j], c),
