@@ -1768,6 +1768,20 @@ hipError_t launch_layer_norm_split(const float* x, int ldx, const float* gamma, 
     return hipGetLastError();
 }
 
+template <int RT, int NW, bool kStage>
+hipError_t run_attention4(const AttnArgs& a, int n_chunks, hipStream_t s)
+{
+    // LDS above the default dynamic limit is granted once per kernel
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&rel_pos_attention4<RT, NW, kStage>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    if (attr != hipSuccess) return attr;
+    const dim3 grid((a.T + 16 * RT - 1) / (16 * RT), a.H, n_chunks);
+    hipLaunchKernelGGL((rel_pos_attention4<RT, NW, kStage>), grid, dim3(64 * NW),
+                       (unsigned)attn_lds_bytes(a.T, RT, NW, kStage), s, a);
+    return hipGetLastError();
+}
+
 // Which attention kernel: by the workgroups that 16 and 32 query rows a
 // workgroup make of the launch (us, one sequence of 8 heads unless said):
 // - up to one 16-row workgroup a CU, its operands staged: 23.5 at T = 416, where
@@ -1789,21 +1803,12 @@ hipError_t launch_attention(const AttnArgs& a, int n_chunks, hipStream_t s)
         hipLaunchKernelGGL(rel_pos_attention_long, grid, dim3(256), 4u * kTileFloats, s, a);
         return hipGetLastError();
     }
-    auto run = [&](auto kern, int rt, int nw, bool stage) {
-        // LDS above the default dynamic limit is granted once per instantiation
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-        if (attr != hipSuccess) return attr;
-        const dim3 grid((a.T + 16 * rt - 1) / (16 * rt), a.H, n_chunks);
-        hipLaunchKernelGGL(kern, grid, dim3(64 * nw), (unsigned)attn_lds_bytes(a.T, rt, nw, stage), s, a);
-        return hipGetLastError();
-    };
     constexpr long long kCus = 256;
     const long long n16 = (long long)((a.T + 15) / 16) * a.H * n_chunks;
     const long long n32 = (long long)((a.T + 31) / 32) * a.H * n_chunks;
-    if (n16 <= kCus || a.T > 1024) return run(rel_pos_attention4<1, 8, true>, 1, 8, true);
-    if (n32 <= kCus) return run(rel_pos_attention4<2, 8, false>, 2, 8, false);
-    return run(rel_pos_attention4<2, 4, false>, 2, 4, false);
+    if (n16 <= kCus || a.T > 1024) return run_attention4<1, 8, true>(a, n_chunks, s);
+    if (n32 <= kCus) return run_attention4<2, 8, false>(a, n_chunks, s);
+    return run_attention4<2, 4, false>(a, n_chunks, s);
 }
 
 size_t attn_fast_ws_floats(int T, int H, int n_chunks)

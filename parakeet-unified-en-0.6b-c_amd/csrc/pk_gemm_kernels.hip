@@ -5,6 +5,8 @@
 #include "pk_gpu.h"
 #include "pk_gemm_tiles.h"
 
+#include <limits>
+
 namespace pkgpu {
 namespace {
 
@@ -136,18 +138,19 @@ int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip = false)
 {
     const double k = K / 1024.0;
     const double w_bytes = (kind == W_F32 ? 4.0 : kind == W_I8 ? 1.0 : 0.625) * K * N;
-    int best = 0;
-    double best_t = 0.0;
+    int best = chain4::kNumTiles - 1;
+    double best_t = std::numeric_limits<double>::infinity();
     const int n = chain4::kNumTiles - (shares_chip ? 1 : 0);
     for (int i = 0; i < n; ++i) {
         const chain4::Chain4Tile& t = chain4::kTiles[i];
-        const long long rows = (M + t.bm - 1) / t.bm, cols = (N + t.bn - 1) / t.bn;
+        const long long rows = ((long long)M + t.bm - 1) / t.bm, cols = ((long long)N + t.bn - 1) / t.bn;
+        if (rows > 65535) continue;                   // the grid's limit; 128 rows a tile reach furthest
         const Rounds& r = kChain4Rounds[kind][i];
         double rounds = (double)((rows * cols + kCus - 1) / kCus);
         if (shares_chip) rounds = std::max(1.0, (double)(rows * cols) / kCus);
         const double compute = r.a + r.b * k + (rounds - 1) * (r.e + r.c * k);
         const double time = std::max(compute, (rows * w_bytes + cols * 4.0 * M * K) / kL2BytesPerUs);
-        if (i == 0 || time < best_t) {
+        if (time < best_t) {
             best = i;
             best_t = time;
         }

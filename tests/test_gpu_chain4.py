@@ -146,6 +146,11 @@ def test_chain_tile_choice():
         assert lib.pk_gpu_pick_chain_tile(16, 1024, 1024, bits) == 0
         assert lib.pk_gpu_pick_chain_tile(3312, 4096, 1024, bits) >= 4
     assert taken == set(TILES)
+    # rows of tiles beyond the grid's 65535 leave only taller tiles (K = 1 tiles: 128 rows)
+    for M, tile_rows in ((16 * 65535 + 1, 17), (64 * 65535 + 1, 65), (8388480, 128)):
+        bm = {0: 16, 1: 32, 2: 48, 3: 64, 4: 64, 5: 128}
+        for N in (16, 32, 64):
+            assert bm[lib.pk_gpu_pick_chain_tile(M, N, 32, 32)] >= tile_rows
     assert lib.pk_gpu_pick_chain_tile(16, 16, 16, 7) == -1 and lib.pk_gpu_pick_chain_tile(0, 16, 16, 8) == -1
     assert lib.pk_gpu_force_chain_tile(len(TILES)) == -1
     assert lib.pk_gpu_force_chain_tile(-1) == 0
