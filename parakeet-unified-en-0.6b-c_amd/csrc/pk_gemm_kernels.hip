@@ -247,8 +247,11 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, 
     a.s_bytes = (uint32_t)s_ext;
     const uintptr_t pa = reinterpret_cast<uintptr_t>(p.A), pb = reinterpret_cast<uintptr_t>(p.B);
     a.vec_a = (p.lda % 4 == 0) && (pa % 16 == 0);
+    // int4 rows are read by words of 8 columns: where N ends inside one, the last
+    // row's word ends past b_bytes, and the descriptor's range check returns 0 for
+    // all of it
     a.vec_b = p.kind == W_F32 ? ((p.ldb % 4 == 0) && (pb % 16 == 0))
-                              : ((p.ldb % 4 == 0) && (pb % 4 == 0));
+                              : ((p.ldb % 4 == 0) && (pb % 4 == 0) && (p.kind != W_I4 || p.N % 8 == 0));
 
     int n_main = p.N;
     if (p.kind == W_I8) n_main = (p.N / 16) * 16;     // blas.c:686, 734

@@ -89,8 +89,8 @@ def test_chain_tile_bit_exact(dev, tile, kind):
 @pytest.mark.parametrize("N", [16, 40, 72, 200])
 @pytest.mark.parametrize("kind", ["f32", "i8", "i4"])
 def test_chain_tile_partial_columns(dev, kind, N):
-    """Columns that end inside a unit of 8, a tile, and (int8) before the edge
-    columns; every epilogue, vector and scalar output rows."""
+    """Columns that end inside a tile, and (int8) before the edge columns; every
+    epilogue, vector output rows (scalar ones: test_chain_tile_scalar_rows)."""
     bias = po.normal((N,), 0.0, 1.0, po.seed(SEED, f"bias.{N}"))
     for tile in TILES:
         for M, K, epi, beta in ((35, 68, pk.EPI_NONE, 0.0), (19, 132, pk.EPI_SWISH, 0.0),
@@ -100,6 +100,77 @@ def test_chain_tile_partial_columns(dev, kind, N):
             got = run(dev, kind, A, W, extra, C0, K, beta, bias, epi, tile=tile)
             want = run(dev, kind, A, W, extra, C0, K, beta, bias, epi, cfg=13)
             assert bits_equal(got, want), f"tile {tile} {kind} {M}x{N}x{K}: {describe_mismatch(got, want)}"
+
+
+def padded(a, ld, rng):
+    """a's rows `ld` elements apart, the elements between them at random."""
+    out = rng.integers(0, 256, (a.shape[0], ld * a.itemsize), dtype=np.uint8).view(a.dtype).reshape(a.shape[0], ld)
+    out[:, :a.shape[1]] = a
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,N", [("f32", 33), ("f32", 37), ("f32", 50), ("i4", 34), ("i4", 44), ("i4", 70),
+                                    ("i4", 72), ("i8", 34), ("i8", 48)])
+def test_chain_tile_scalar_rows(dev, kind, N):
+    """Weight rows padded to whole words, with columns that end inside a unit of
+    8 (f32: a part of it lies past the last row's end; i4: not for the four-deep
+    tiles, whichever is forced) and output rows that allow no vector stores: an
+    odd row stride, C and bias off their alignment by one float.  Every tile and
+    the K = 1 kernels against the oracle; nothing beside the columns is written."""
+    rng = np.random.default_rng(N)
+    guard = np.float32(-7.0)
+    for tile, cfg in [(t, -1) for t in TILES] + [(-1, 13), (-1, 20)]:
+        for i, (M, K, epi, beta, ldc, off) in enumerate((
+                (35, 68, pk.EPI_NONE, 0.5, N + 1, 0), (17, 131, pk.EPI_SWISH, 0.0, N + 3, 1),
+                (70, 96, pk.EPI_HALF_RESIDUAL, 0.0, N + 4 - N % 4, 1), (5, 40, pk.EPI_RESIDUAL, 0.0, N + 1, 0),
+                (129, 64, EPI_RELU, 1.0, N + 4 - N % 4, 0), (33, 33, pk.EPI_NONE, 1.0, N + 5, 1))):
+            A, W, extra, C0 = make(kind, M, N, K, f"sr.{kind}.{M}.{N}.{K}")
+            bias = po.normal((N,), 0.0, 1.0, po.seed(SEED, f"sr.bias.{N}")) if i % 2 == 0 or epi else None
+            ldb = (W.shape[1] + 3) // 4 * 4 + 4 * (i % 2)
+            a, w = dev.put(A), dev.put(padded(W, ldb, rng))
+            s = dev.put(extra) if kind == "i4" else None
+            c = dev.torch.full((off + M * ldc,), float(guard), device=dev.dev)
+            cv = c[off:].view(M, ldc)
+            cv[:, :N] = dev.put(C0)
+            b = dev.torch.zeros(N + 1, device=dev.dev)
+            if bias is not None:
+                b[off:off + N] = dev.put(bias)
+            pk.call("pk_gpu_set_numerics", pk.NUMERICS_EXACT)
+            pk.call("pk_gpu_force_config", cfg)
+            pk.call("pk_gpu_force_chain_tile", tile)
+            try:
+                tail = (beta, cv.data_ptr(), ldc, b[off:].data_ptr() if bias is not None else None, epi, dev.stream())
+                if kind == "i4":
+                    pk.call("pk_gpu_gemm_i4_ex_dev", M, N, K, 1.0, a.data_ptr(), A.shape[1], w.data_ptr(),
+                            s.data_ptr(), ldb, *tail)
+                elif kind == "i8":
+                    pk.call("pk_gpu_gemm_i8_ex_dev", M, N, K, 1.0, a.data_ptr(), A.shape[1], w.data_ptr(), extra, ldb,
+                            *tail)
+                else:
+                    pk.call("pk_gpu_sgemm_ex_dev", M, N, K, 1.0, a.data_ptr(), A.shape[1], w.data_ptr(), ldb, *tail)
+            finally:
+                pk.call("pk_gpu_force_chain_tile", -1)
+                pk.call("pk_gpu_force_config", -1)
+                pk.call("pk_gpu_set_numerics", pk.NUMERICS_DEFAULT)
+            dev.sync()
+            got = c.cpu().numpy()
+            want = oracle(kind, A, W, extra, C0, K, beta)
+            if bias is not None:
+                want = want + bias
+            if epi == pk.EPI_SWISH:
+                want = po.swish(want)
+            elif epi == pk.EPI_HALF_RESIDUAL:                   # fma: the half is exact
+                want = np.float32(0.5) * want + C0
+            elif epi == pk.EPI_RESIDUAL:
+                want = C0 + want
+            elif epi == EPI_RELU:
+                want = np.where(want > 0, want, np.float32(0.0))
+            rows = got[off:].reshape(M, ldc)
+            what = f"tile {tile} config {cfg} {kind} {M}x{N}x{K} ldc {ldc}"
+            assert (got[:off] == guard).all() and (rows[:, N:] == guard).all(), what
+            cols = np.ascontiguousarray(rows[:, :N])
+            assert bits_equal(cols, want), f"{what}: {describe_mismatch(cols, want)}"
 
 
 @pytest.mark.gpu
