@@ -111,6 +111,11 @@ int pkor_encoder_run(const void *blocks, int n_blocks, const float *pe_table, in
                      int pe_center, const float *x, int T, int chunk, int overlap, float *out,
                      float *snapshots);
 
+/* pre_encode_and_scale (encoder.c:103-174, 578-592): mel [128][n_frames] with
+ * the weights of a pk_gpu_pre_encode_weights (include/pk_gpu.h) to out
+ * [T'][1024].  Returns T', or -1 on a bad argument or no memory. */
+int pkor_pre_encode(const void *weights, const float *mel, int n_frames, float *out);
+
 #ifdef __cplusplus
 }
 #endif

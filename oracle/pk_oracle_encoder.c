@@ -1,5 +1,6 @@
-/*  pk_oracle_encoder.c - CPU oracle of the whole encoder: the 24 conformer
- *  blocks over a chunked input, composed of the oracle's pinned operations.
+/*  pk_oracle_encoder.c - CPU oracle of the whole encoder: the pre-encode
+ *  (at the end of this file) and the 24 conformer blocks over a chunked
+ *  input, composed of the oracle's pinned operations.
  *
  *  TEST INFRASTRUCTURE ONLY (see pk_oracle.h).  Built with -ffp-contract=off
  *  so every rounding happens as written; fused steps use fmaf().
@@ -260,5 +261,89 @@ int pkor_encoder_run(const void *blocks_v, int n_blocks, const float *pe_table, 
     rc = 0;
 done:
     free(ch); free(xs); free(ln); free(h); free(att); free(P); free(cm); free(cm2);
+    return rc;
+}
+
+/* ---- pre-encode --------------------------------------------------------- */
+
+/* pre_encode_and_scale (encoder.c:103-174, 578-592), every convolution
+ * [channel][H][W] as pk_conv2d (tensor_ops.c:436-475) computes it: an output
+ * starts from its bias and takes v = fma(x, w, v) over its in-range taps,
+ * (ic, kh, kw) ascending.  Image row t is mel frame t, column f is mel bin f.
+ *   conv.0 1 -> 256, 3x3, stride 2, pad 1, ReLU
+ *   conv.2 depthwise 3x3, stride 2, pad 1;  conv.3 256 -> 256, 1x1, ReLU
+ *   conv.5 depthwise 3x3, stride 2, pad 1;  conv.6 256 -> 256, 1x1, ReLU
+ *   row t flattened to c * W + f (encoder.c:152-158); out linear + bias, * 32
+ * ReLU is max(v, 0) as _mm256_max_ps(v, 0) gives it: v if v > 0, else +0. */
+enum { SUB = 256, MELS = 128 };
+
+static float relu(float v) { return v > 0.0f ? v : 0.0f; }
+
+static int half_up(int n) { return (n - 1) / 2 + 1; }
+
+/* 3x3, stride 2, pad 1: output channel c from plane `c * plane` of in (plane 0:
+ * one input channel for all). */
+static void conv3x3s2(const float *in, size_t plane, int H, int W, const float *w, const float *b,
+                      int with_relu, float *out)
+{
+    const int Ho = half_up(H), Wo = half_up(W);
+    #pragma omp parallel for
+    for (int c = 0; c < SUB; c++)
+        for (int oh = 0; oh < Ho; oh++)
+            for (int ow = 0; ow < Wo; ow++) {
+                float v = b[c];
+                for (int kh = 0; kh < 3; kh++)
+                    for (int kw = 0; kw < 3; kw++) {
+                        const int ih = 2 * oh - 1 + kh, iw = 2 * ow - 1 + kw;
+                        if (ih < 0 || ih >= H || iw < 0 || iw >= W) continue;
+                        v = fmaf(in[c * plane + (size_t)ih * W + iw], w[c * 9 + kh * 3 + kw], v);
+                    }
+                out[((size_t)c * Ho + oh) * Wo + ow] = with_relu ? relu(v) : v;
+            }
+}
+
+/* 1x1, 256 -> 256 over n positions, ReLU. */
+static void conv1x1(const float *in, int n, const float *w, const float *b, float *out)
+{
+    #pragma omp parallel for
+    for (int c = 0; c < SUB; c++) {
+        float *o = out + (size_t)c * n;
+        for (int i = 0; i < n; i++) o[i] = b[c];
+        for (int ic = 0; ic < SUB; ic++) {
+            const float *x = in + (size_t)ic * n;
+            const float wv = w[c * SUB + ic];
+            for (int i = 0; i < n; i++) o[i] = fmaf(x[i], wv, o[i]);
+        }
+        for (int i = 0; i < n; i++) o[i] = relu(o[i]);
+    }
+}
+
+int pkor_pre_encode(const void *weights, const float *mel, int n_frames, float *out)
+{
+    const pk_gpu_pre_encode_weights *w = (const pk_gpu_pre_encode_weights *)weights;
+    if (n_frames <= 0) return -1;
+    const int H1 = half_up(n_frames), W1 = half_up(MELS), H2 = half_up(H1), W2 = half_up(W1);
+    const int H3 = half_up(H2), W3 = half_up(W2), F = SUB * W3;
+    float *img = (float *)malloc((size_t)n_frames * MELS * sizeof(float));
+    float *a = (float *)malloc((size_t)SUB * H1 * W1 * sizeof(float));
+    float *b = (float *)malloc((size_t)SUB * H2 * W2 * sizeof(float));
+    float *lin = weight_f32(&w->out_w, F, D_MODEL);
+    int rc = -1;
+    if (img && a && b && lin) {
+        for (int t = 0; t < n_frames; t++)
+            for (int f = 0; f < MELS; f++) img[(size_t)t * MELS + f] = mel[(size_t)f * n_frames + t];
+        conv3x3s2(img, 0, n_frames, MELS, w->conv0_w, w->conv0_b, 1, a);
+        conv3x3s2(a, (size_t)H1 * W1, H1, W1, w->conv2_w, w->conv2_b, 0, b);
+        conv1x1(b, H2 * W2, w->conv3_w, w->conv3_b, a);
+        conv3x3s2(a, (size_t)H2 * W2, H2, W2, w->conv5_w, w->conv5_b, 0, b);
+        conv1x1(b, H3 * W3, w->conv6_w, w->conv6_b, a);
+        for (int t = 0; t < H3; t++)
+            for (int c = 0; c < SUB; c++)
+                memcpy(b + (size_t)t * F + (size_t)c * W3, a + ((size_t)c * H3 + t) * W3, W3 * sizeof(float));
+        gemm_chain(H3, D_MODEL, F, b, F, lin, w->out_b, EPI_NONE, out, D_MODEL);
+        for (size_t i = 0; i < (size_t)H3 * D_MODEL; i++) out[i] *= 32.0f;
+        rc = H3;
+    }
+    free(img); free(a); free(b); free(lin);
     return rc;
 }

@@ -87,6 +87,8 @@ def oracle():
         lib.pkor_depthwise_conv1d.argtypes = [_p, _p, _p, _p, _i, _i, _i]
         lib.pkor_encoder_run.argtypes = [_p, _i, _p, _i, _i, _p, _i, _i, _i, _p, _p]
         lib.pkor_encoder_run.restype = _i
+        lib.pkor_pre_encode.argtypes = [_p, _p, _i, _p]
+        lib.pkor_pre_encode.restype = _i
         for fn in (lib.pkor_layer_norm_rows, lib.pkor_softmax_rows, lib.pkor_attention_core,
                    lib.pkor_glu_rows, lib.pkor_depthwise_conv1d):
             fn.restype = None
@@ -374,6 +376,18 @@ def ref_pre_encode(w, mel, variant="portable"):
     got = lib.pkref_pre_encode(ctypes.byref(w), _ptr(mel), n, _ptr(out))
     if got != tp:
         raise RuntimeError(f"pkref_pre_encode returned {got}, expected {tp}")
+    return out
+
+
+def pre_encode(w, mel):
+    """The oracle's pre_encode_and_scale (pk_oracle_encoder.c), arguments and
+    result as ref_pre_encode's."""
+    mel = _f32(mel)
+    n = mel.shape[1]
+    tp = (((n - 1) // 2 + 1 - 1) // 2 + 1 - 1) // 2 + 1
+    out = np.empty((tp, 1024), np.float32)
+    if oracle().pkor_pre_encode(ctypes.byref(w), _ptr(mel), n, _ptr(out)) != tp:
+        raise RuntimeError("pkor_pre_encode failed")
     return out
 
 

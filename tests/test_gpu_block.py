@@ -430,6 +430,61 @@ def test_pre_encode_bit_exact(dev, enc2, out_bits):
         assert bits_equal(got, want), f"n_frames={n}: " + describe_mismatch(got, want)
 
 
+# mel frames: 1 to 3 rows at every stage, and around the edges of the 16 frames
+# (4 rows of conv.2) that a workgroup of conv0_conv2 takes, whose first and last
+# rows and columns leave taps of conv.0 and conv.2 outside the image; 128 bins
+# are 4 blocks of 8 columns
+PRE_FRAMES = [1, 2, 3, 4, 5, 7, 8, 9, 12, 13, 14, 15, 16, 17, 18, 19, 20, 29, 31, 32, 33, 47, 48, 49, 50, 63, 64,
+              65, 127, 130, 509]
+
+
+@pytest.mark.parametrize("out_bits", [8, 32])
+def test_pre_encode_bit_exact_to_oracle(dev, enc2, out_bits):
+    """conv0_conv2, conv.5, the flatten and the GEMMs between them against the
+    CPU oracle; nothing is written past T' rows."""
+    pre = bg.PreEncode(0xB10D5 + out_bits, out_bits)
+    pk.call("pk_gpu_encoder_set_pre_encode", enc2.h, ctypes.byref(pre.w))
+    lib = pk.load()
+    for n in PRE_FRAMES:
+        mel = rows(128, n, 2.0)
+        want = po.pre_encode(pre.w, mel)
+        tp = lib.pk_gpu_encoder_frames(n)
+        assert tp == want.shape[0]
+        dmel = dev.put(mel)
+        dx = dev.torch.full((tp + 1, 1024), -7.0, device=dev.dev)
+        pk.call("pk_gpu_encoder_pre_encode_dev", enc2.h, dmel.data_ptr(), n, dx.data_ptr(), dev.stream())
+        got = dx.cpu().numpy()
+        assert (got[tp:] == -7.0).all()
+        assert bits_equal(got[:tp], want), f"n_frames={n}: " + describe_mismatch(got[:tp], want)
+
+
+def test_pre_encode_edges_reach_the_output(dev, enc2):
+    """A mel spectrogram that is zero but for its first or last frame or bin:
+    what the edge taps of the fused convolutions contribute, bit for bit."""
+    pre = bg.PreEncode(0xB10D7)
+    pk.call("pk_gpu_encoder_set_pre_encode", enc2.h, ctypes.byref(pre.w))
+    for n in (16, 17, 34):
+        for part in (np.s_[:, 0], np.s_[:, n - 1], np.s_[0, :], np.s_[127, :], np.s_[:, 15], np.s_[31:34, :]):
+            mel = np.zeros((128, n), np.float32)
+            mel[part] = rows(128, n, 2.0)[part]
+            want = po.pre_encode(pre.w, mel)
+            dmel, dx = dev.put(mel), dev.torch.empty(want.shape, device=dev.dev)
+            pk.call("pk_gpu_encoder_pre_encode_dev", enc2.h, dmel.data_ptr(), n, dx.data_ptr(), dev.stream())
+            got = dx.cpu().numpy()
+            assert bits_equal(got, want), f"n_frames={n} {part}: " + describe_mismatch(got, want)
+
+
+def test_run_mel_equals_oracle_pre_encode_then_blocks(dev, enc2):
+    """pk_gpu_encoder_run_mel = the oracle's pre-encode, then the blocks."""
+    pre = bg.PreEncode(0xB10D8)
+    pk.call("pk_gpu_encoder_set_pre_encode", enc2.h, ctypes.byref(pre.w))
+    n = 3300                                        # T' = 413 -> two chunks
+    mel = rows(128, n, 2.0)
+    out = np.empty((pk.load().pk_gpu_encoder_frames(n), 1024), np.float32)
+    pk.call("pk_gpu_encoder_run_mel", enc2.h, mel.ctypes.data, n, 400, 8, out.ctypes.data)
+    assert bits_equal(out, enc2.run(po.pre_encode(pre.w, mel), chunk=400))
+
+
 @pytest.mark.skipif(not po.have_ref_block(), reason="reference block harness missing")
 def test_run_mel_equals_pre_encode_then_blocks(dev, enc2):
     """pk_gpu_encoder_run_mel = pre-encode on the device, then the blocks

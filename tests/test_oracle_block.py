@@ -330,3 +330,57 @@ def test_encoder_oracle_thread_count_invariant():
         assert out.returncode == 0, out.stderr[-2000:]
         digests.add(out.stdout.strip())
     assert len(digests) == 1
+
+
+def pre_encode_f64(p, mel):
+    """The pre-encode in 64 bits with torch's convolutions; p: a blockgen.PreEncode."""
+    import ctypes
+    import torch
+    F = torch.nn.functional
+
+    def arr(ptr, shape, ct=ctypes.c_float):
+        return torch.from_numpy(np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(ct)), shape).copy()).double()
+
+    def conv(x, n, groups):
+        w = arr(getattr(p.w, n + "_w"), (256, 1, 3, 3))
+        return F.conv2d(x, w, arr(getattr(p.w, n + "_b"), (256,)), stride=2, padding=1, groups=groups)
+
+    def point(x, n):
+        w = arr(getattr(p.w, n + "_w"), (256, 256, 1, 1))
+        return torch.relu(F.conv2d(x, w, arr(getattr(p.w, n + "_b"), (256,))))
+
+    x = torch.relu(conv(torch.from_numpy(mel).t()[None, None].double(), "conv0", 1))
+    x = point(conv(x, "conv2", 256), "conv3")
+    x = point(conv(x, "conv5", 256), "conv6")[0]                  # [256][T'][16]
+    x = x.permute(1, 0, 2).reshape(x.shape[1], -1)
+    ow = p.w.out_w
+    if ow.bits == 8:
+        w = arr(ow.data, (4096, 1024), ctypes.c_int8) * float(np.float32(ow.scale))
+    else:
+        w = arr(ow.data, (4096, 1024))
+    return ((x @ w + arr(p.w.out_b, (1024,))) * 32.0).numpy()
+
+
+@pytest.mark.parametrize("out_bits", [8, 32])
+@pytest.mark.parametrize("n", [1, 2, 9, 40, 131])
+def test_pre_encode_oracle_closed_form(n, out_bits):
+    """Against the same network in 64 bits.  No output has more than 4096 + 2 *
+    (256 + 9) + 9 roundings of 2^-24 on its way, which add up like a random walk:
+    about 70 of them, and 2^-17 of the result covers it."""
+    import blockgen as bg
+    p = bg.PreEncode(0xB10CE + out_bits, out_bits)
+    mel = rows(128, n, 2.0)
+    got, want = po.pre_encode(p.w, mel), pre_encode_f64(p, mel)
+    assert got.shape == want.shape
+    assert np.linalg.norm(got - want) <= 2.0 ** -17 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 2.0 ** -15 * np.abs(want).max()
+
+
+@pytest.mark.skipif(not po.have_ref_block(), reason="reference block harness missing")
+@pytest.mark.parametrize("out_bits", [8, 32])
+def test_pre_encode_oracle_bit_exact_to_reference(out_bits):
+    import blockgen as bg
+    p = bg.PreEncode(0xB10CE + out_bits, out_bits)
+    for n in (1, 8, 33, 100, 401):
+        mel = rows(128, n, 2.0)
+        assert bits_equal(po.pre_encode(p.w, mel), po.ref_pre_encode(p.w, mel)), n
