@@ -317,8 +317,9 @@ int pk_gpu_encoder_run(pk_gpu_encoder *enc, const float *x, int T, int chunk_siz
  * that call, so they never overlap.  One encoder takes calls from one host
  * thread at a time.  The blocks'
  * launches are captured in a HIP graph on the first run of each (T,
- * chunk_size, overlap, configuration forced with pk_gpu_force_config on the
- * calling thread) and replayed afterwards (not while profiling). */
+ * chunk_size, overlap, configuration and tile forced with pk_gpu_force_config
+ * and pk_gpu_force_chain_tile on the calling thread) and replayed afterwards
+ * (not while profiling). */
 int pk_gpu_encoder_run_dev(pk_gpu_encoder *enc, const float *dx, int T, int chunk_size,
                            int overlap, float *dout, void *stream);
 /* Pre-encode parameters (PreEncodeWeights, parakeet.h), host pointers:
@@ -353,6 +354,8 @@ int pk_gpu_encoder_run_mel(pk_gpu_encoder *enc, const float *mel, int n_frames, 
 
 /* Device bytes held by the encoder (weights + workspace). */
 size_t pk_gpu_encoder_bytes(const pk_gpu_encoder *enc);
+/* HIP graphs the encoder holds (pk_gpu_encoder_run_dev). */
+int pk_gpu_encoder_graphs(const pk_gpu_encoder *enc);
 
 /* Per-stage timing of later runs: with enable != 0, every launch of a run is
  * bracketed by HIP events on the caller's stream (the reference's pk_verbose
@@ -574,7 +577,8 @@ int pk_gpu_force_config(int index);
 /* The exact GEMMs' own tiles (16-byte aligned rows, alpha = 1): their number,
  * the one that a shape with weights of `bits` = 4, 8 or 32 bits takes (-1:
  * invalid), and a test hook that forces one for later GEMM calls on this
- * thread (-1 = automatic).  The tile never changes a result. */
+ * thread (-1 = automatic).  The tile never changes a result.  A resident
+ * encoder keeps a graph per forced tile, as for pk_gpu_force_config. */
 int pk_gpu_num_chain_tiles(void);
 int pk_gpu_pick_chain_tile(int M, int N, int K, int bits);
 int pk_gpu_force_chain_tile(int tile);

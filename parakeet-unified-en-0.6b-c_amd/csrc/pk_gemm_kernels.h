@@ -123,6 +123,8 @@ struct TileConfig {
 // forced configurations and what the four-deep chains (pk_chain4.h) do not
 // take: alpha other than 1, and operands whose rows allow no vector loads.
 int choose_config_index(int M, int N, int K, WeightKind kind);
+// The calling thread's pk_gpu_force_chain_tile tile (-1: the rule picks).
+int forced_chain_tile();
 // Number of configurations and access by index (for tests and sweeps).
 int num_configs();
 TileConfig config_at(int i);

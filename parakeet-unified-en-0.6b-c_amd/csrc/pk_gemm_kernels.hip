@@ -159,6 +159,7 @@ int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip = false)
 }
 }  // namespace
 
+int forced_chain_tile() { return t_chain_tile; }
 
 hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, Tolerance tol)
 {

@@ -129,11 +129,12 @@ struct pk_gpu_encoder {
     // the 24 blocks' launches captured once per (T, chunk, overlap) and
     // replayed; their device pointers are the workspace's, so a workspace
     // change drops them
-    // (T, chunk, overlap, group, forced tile config): a graph freezes the
-    // tiles its GEMMs were launched with, so a pk_gpu_force_config in force
-    // at capture is part of what the graph is
+    // (T, chunk, overlap, group, forced tile config, forced exact tile): a
+    // graph freezes the tiles its GEMMs were launched with, so a
+    // pk_gpu_force_config or pk_gpu_force_chain_tile in force at capture is
+    // part of what the graph is
     // and the encoder's numerics (which kernels its GEMMs take)
-    std::map<std::tuple<int, int, int, int, int, int>, hipGraphExec_t> graphs;
+    std::map<std::tuple<int, int, int, int, int, int, int>, hipGraphExec_t> graphs;
     int numerics = PK_GPU_NUMERICS_EXACT;     // pk_gpu_encoder_set_numerics
     // Row groups replayed concurrently: group 0 on the caller's stream, group
     // g > 0 on side[g - 1], joined through events around the replay.
@@ -1054,14 +1055,14 @@ int run_queued(pk_gpu_encoder* e, const float* x, int T, int chunk, int ov, floa
         // encoder's own stream (the null stream cannot capture).  A caller
         // that sees many input lengths would keep adding graphs; past
         // kMaxGraphs they are all dropped and recaptured on demand.
-        const int forced = pkgpu::rt::forced_config();
+        const int forced = pkgpu::rt::forced_config(), forced_tile = pkgpu::forced_chain_tile();
         // The other groups start when group 0 has run the first `lag` modules
         // of block 0 (its lead graph), so that the groups' GEMMs and their
         // row kernels fall at different times.
         const int lag = groups.size() < 2 ? 0 : e->lag >= 0 ? e->lag : group_lag();
         if (e->graphs.size() + groups.size() + (lag > 0) > kMaxGraphs &&
             !e->graphs.count(std::make_tuple(T, chunk, ov, lag > 0 ? 100 + lag : 0, forced,
-                                             e->numerics))) {
+                                             forced_tile, e->numerics))) {
             if ((rc = check(hipStreamSynchronize(s), "encoder stream"))) return rc;
             for (hipStream_t st : e->side)
                 if ((rc = check(hipStreamSynchronize(st), "encoder stream"))) return rc;
@@ -1069,7 +1070,7 @@ int run_queued(pk_gpu_encoder* e, const float* x, int T, int chunk, int ov, floa
         }
         auto graph = [&](int id, int gi, int b_from, int m_from, int b_to, int m_to,
                          hipGraphExec_t* out) -> int {
-            const auto key = std::make_tuple(T, chunk, ov, id, forced, e->numerics);
+            const auto key = std::make_tuple(T, chunk, ov, id, forced, forced_tile, e->numerics);
             auto it = e->graphs.find(key);
             if (it == e->graphs.end()) {
                 int r = check(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal),
@@ -1358,6 +1359,8 @@ size_t pk_gpu_encoder_bytes(const pk_gpu_encoder* enc)
                      enc->panel_bytes + enc->split_bytes
                : 0;
 }
+
+int pk_gpu_encoder_graphs(const pk_gpu_encoder* enc) { return enc ? (int)enc->graphs.size() : 0; }
 
 int pk_gpu_encoder_profile(pk_gpu_encoder* enc, int enable)
 {

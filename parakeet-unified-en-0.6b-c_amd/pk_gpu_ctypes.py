@@ -45,6 +45,7 @@ _PROTOS = {
     "pk_gpu_pick_config": (_i, [_i, _i, _i]),
     "pk_gpu_pick_config_bits": (_i, [_i, _i, _i, _i]),
     "pk_gpu_force_config": (_i, [_i]),
+    "pk_gpu_encoder_graphs": (_i, [_p]),
     "pk_gpu_num_chain_tiles": (_i, []),
     "pk_gpu_pick_chain_tile": (_i, [_i, _i, _i, _i]),
     "pk_gpu_force_chain_tile": (_i, [_i]),

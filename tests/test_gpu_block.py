@@ -337,6 +337,27 @@ def test_encoder_forced_config_is_part_of_the_graph(dev, enc2):
             pk.call("pk_gpu_force_config", -1)
 
 
+def test_encoder_forced_chain_tile_is_part_of_the_graph(dev, enc2):
+    """Likewise pk_gpu_force_chain_tile: a run under another forced tile
+    captures graphs of its own, one under a tile seen before finds them, and
+    every tile gives the same bits."""
+    T, lib = 892, pk.load()                     # a length no other test captures
+    x = rows(T, 1024)
+    want = enc2.run(x, chunk=400)
+    seen = {-1: lib.pk_gpu_encoder_graphs(enc2.h)}
+    for tile in (0, 4, -1, 0):
+        pk.call("pk_gpu_force_chain_tile", tile)
+        try:
+            before = lib.pk_gpu_encoder_graphs(enc2.h)
+            for _ in range(2):                  # capture (or reuse), then replay
+                assert bits_equal(enc2.run(x, chunk=400), want), f"forced tile {tile}"
+            captured = lib.pk_gpu_encoder_graphs(enc2.h) - before
+        finally:
+            pk.call("pk_gpu_force_chain_tile", -1)
+        assert (captured == 0) == (tile in seen), f"forced tile {tile}: {captured} graphs captured"
+        seen[tile] = 1
+
+
 @pytest.mark.parametrize("n_groups", [1, 2, 3, 4])
 def test_encoder_row_groups_are_bit_identical(dev, enc2, n_groups):
     """Replays split the chunks into row groups replayed concurrently (group 0
