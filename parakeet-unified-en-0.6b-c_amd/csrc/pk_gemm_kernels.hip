@@ -117,19 +117,32 @@ namespace {
 // 2000 x 1024 x 4096 fp32 (2.1 GB of operands) take 183 us instead of the 133 of
 // their rounds, 64 x 64 ones 131.
 //
+// Below K = 1024 the ends of a round weigh more, and small tiles pay more for
+// theirs than the fit above says, large ones hide them under each other: from
+// round kEndsFrom on (of the small tiles a CU holds three or four workgroups at
+// once, which start together) e goes to e0 at K = 0, fitted at K = 64..640 to M =
+// 16..204800, N = 64..4096.  There the pick takes 1 % more than the best tile on
+// average; without e0 25 % more at K = 64 and 5 % at K = 256, and up to 1.8 times
+// the K = 1 kernels' time (204800 x 1024 x 64 fp32: 713 us on 32 x 32 tiles, 400
+// on 64 x 64, K = 1 391; 204800 x 256 x 256 int4: 332, 240, 266).
+//
 // shares_chip: other kernels run beside the GEMM and take what its last round
 // leaves free, so a part of a round counts as that part; and 128 x 64 tiles, one
 // workgroup of whose registers fill a CU, are left out.  3200 frames in two row
 // groups: 38.2 ms with each GEMM's own best tile, 37.1 so (37.9 with 128 x 64).
-struct Rounds { float a, b, e, c; };
+struct Rounds { float a, b, e, c, e0; };
 constexpr Rounds kChain4Rounds[3][chain4::kNumTiles] = {
-    /* fp32 */ {{2.9f, 3.9f, 0.1f, 3.75f}, {2.8f, 4.3f, 0.2f, 4.0f}, {3.2f, 7.3f, 0.5f, 6.9f},
-                {3.7f, 7.7f, 0.9f, 7.1f}, {4.8f, 14.8f, 1.7f, 14.0f}, {6.3f, 29.9f, 4.0f, 27.6f}},
-    /* int8 */ {{2.9f, 3.9f, 0.3f, 3.9f}, {3.2f, 5.9f, 0.3f, 4.4f}, {3.0f, 8.0f, 0.6f, 7.2f},
-                {4.0f, 9.2f, 1.2f, 7.7f}, {5.0f, 17.0f, 1.5f, 14.7f}, {6.2f, 31.8f, 3.0f, 29.0f}},
-    /* int4 */ {{2.9f, 3.8f, 0.5f, 4.0f}, {3.2f, 6.0f, 0.2f, 4.5f}, {2.5f, 8.2f, 0.4f, 7.2f},
-                {3.3f, 9.8f, 1.1f, 7.8f}, {4.7f, 17.6f, 2.3f, 14.5f}, {5.7f, 32.3f, 4.0f, 28.5f}},
+    /* fp32 */ {{2.9f, 3.9f, 0.1f, 3.75f, 0.76f}, {2.8f, 4.3f, 0.2f, 4.0f, 0.65f},
+                {3.2f, 7.3f, 0.5f, 6.9f, 1.49f}, {3.7f, 7.7f, 0.9f, 7.1f, 1.11f},
+                {4.8f, 14.8f, 1.7f, 14.0f, 0.85f}, {6.3f, 29.9f, 4.0f, 27.6f, 2.34f}},
+    /* int8 */ {{2.9f, 3.9f, 0.3f, 3.9f, 0.74f}, {3.2f, 5.9f, 0.3f, 4.4f, 0.58f},
+                {3.0f, 8.0f, 0.6f, 7.2f, 1.52f}, {4.0f, 9.2f, 1.2f, 7.7f, 0.97f},
+                {5.0f, 17.0f, 1.5f, 14.7f, 0.89f}, {6.2f, 31.8f, 3.0f, 29.0f, 2.57f}},
+    /* int4 */ {{2.9f, 3.8f, 0.5f, 4.0f, 0.75f}, {3.2f, 6.0f, 0.2f, 4.5f, 0.61f},
+                {2.5f, 8.2f, 0.4f, 7.2f, 1.15f}, {3.3f, 9.8f, 1.1f, 7.8f, 1.02f},
+                {4.7f, 17.6f, 2.3f, 14.5f, 0.81f}, {5.7f, 32.3f, 4.0f, 28.5f, 2.66f}},
 };
+constexpr int kEndsFrom[chain4::kNumTiles] = {3, 4, 3, 3, 1, 1};
 constexpr int kCus = 256;
 constexpr double kL2BytesPerUs = 12e6;
 thread_local int t_chain_tile = -1;
@@ -148,7 +161,8 @@ int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip = false)
         const Rounds& r = kChain4Rounds[kind][i];
         double rounds = (double)((rows * cols + kCus - 1) / kCus);
         if (shares_chip) rounds = std::max(1.0, (double)(rows * cols) / kCus);
-        const double compute = r.a + r.b * k + (rounds - 1) * (r.e + r.c * k);
+        double compute = r.a + r.b * k + (rounds - 1) * (r.e + r.c * k);
+        if (k < 1.0) compute += std::max(0.0, rounds - kEndsFrom[i]) * (r.e0 - r.e) * (1.0 - k);
         const double time = std::max(compute, (rows * w_bytes + cols * 4.0 * M * K) / kL2BytesPerUs);
         if (time < best_t) {
             best = i;
@@ -260,9 +274,11 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index, 
 
     hipError_t err = hipSuccess;
     if (n_main > 0 && cfg_index < 0 && a.vec_a && a.vec_b && a.alpha == 1.0f) {
-        // The four-deep chains: the same bits, faster at every size measured.
-        // They read whole vectors and take A as it is; other operands stay on
-        // the K = 1 tiles.
+        // The four-deep chains: the same bits, and over 1038 shapes (M = 16..204800,
+        // N = 64..4096, K = 64..4096, all formats) 0.86 of the K = 1 tiles' time; at
+        // most 5 % more than theirs, but for launches of under 9 us with K = 64 or 128
+        // (up to 13 %).  They read whole vectors and take A as it is; other operands
+        // stay on the K = 1 tiles.
         const int tile = t_chain_tile >= 0 ? t_chain_tile : chain4_pick(p.M, n_main, p.K, p.kind, p.shares_chip);
         switch (p.kind) {
         case W_F32: err = chain4::launch_f32(tile, a, stream); break;
