@@ -78,6 +78,7 @@ struct RowGroup {
     std::map<int, std::pair<int, int>> by_len;
     size_t scores_off = 0;      // its attention's score rows (Tmax > kAttnMaxT) in e->scores
     float* part = nullptr;      // its split-K partial tiles (fast numerics), or null
+    bool shares_chip = false;   // other groups of the run replay beside it
 };
 
 constexpr int kMels = 128;        // PK_N_MELS
@@ -139,7 +140,6 @@ struct pk_gpu_encoder {
     // Row groups replayed concurrently: group 0 on the caller's stream, group
     // g > 0 on side[g - 1], joined through events around the replay.
     int n_groups = 2;
-    bool several_groups = false;        // the current run's row groups are more than one
     int lag = -1;                  // pk_gpu_encoder_set_group_lag (-1: group_lag())
     // fast numerics: LayerNorms feeding a GEMM write pre-split output
     // (PK_GPU_PRESPLIT=0 at creation turns it off; the results are the same)
@@ -524,13 +524,13 @@ std::vector<Chunk> plan_chunks(int T, int C, int ov)
 }
 
 // A weight GEMM of the block: M rows of A through w, with its epilogue;
-// `work`: the row group's split-K partial tiles, or null; `presplit`: A holds
-// a split-output LayerNorm's rows (layer_norm with split); `exact`: the
-// exact chains whatever the encoder's numerics; `ln`: LayerNorms fused into
-// it (fusable() said the panel kernels take them).
+// `g`: the row group it is part of, or null: alone on the chip, on the exact
+// chains whatever the encoder's numerics; `presplit`: A holds a split-output
+// LayerNorm's rows (layer_norm with split); `ln`: LayerNorms fused into it
+// (fusable() said the panel kernels take them).
 int gemm(pk_gpu_encoder* e, const DevWeight& w, const float* A, int M, float* C,
-         const float* bias, Epilogue epi, hipStream_t s, float* work = nullptr,
-         bool presplit = false, bool exact = false, const FusedLn& ln = FusedLn())
+         const float* bias, Epilogue epi, hipStream_t s, const RowGroup* g,
+         bool presplit = false, const FusedLn& ln = FusedLn())
 {
     const double flops = 2.0 * M * w.N * w.K;
     double bytes = weight_bytes_of(w) + 4.0 * M * w.K + 4.0 * M * w.N;
@@ -539,11 +539,11 @@ int gemm(pk_gpu_encoder* e, const DevWeight& w, const float* A, int M, float* C,
     if (ln.in_g) bytes += 8.0 * w.K;
     if (ln.out_g) bytes += 8.0 * w.N;
     if (ln.next_g) bytes += 8.0 * w.N + 4.0 * M * w.N;
-    const pkgpu::Tolerance tol = exact ? pkgpu::TOL_NONE : pkgpu::rt::tolerance_of(e->numerics);
+    const pkgpu::Tolerance tol = g ? pkgpu::rt::tolerance_of(e->numerics) : pkgpu::TOL_NONE;
     return timed(e, stage_of(w), flops, bytes, s,
                  [&] {
-                     GemmProblem p = block_problem(w, A, M, C, bias, epi, tol, work, presplit, ln);
-                     p.shares_chip = e->several_groups;
+                     GemmProblem p = block_problem(w, A, M, C, bias, epi, tol, g ? g->part : nullptr, presplit, ln);
+                     p.shares_chip = g && g->shares_chip;
                      return pkgpu::rt::gemm(p, s, tol);
                  });
 }
@@ -682,8 +682,8 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
         const FusedLn f = fused_in(w1, gm, be, h, b1, pkgpu::EPI_SWISH);
         const float* A = nullptr;
         int r = norm_in(f, gm, be, &A, ready);
-        if (!r) r = gemm(e, w1, A, R, h, b1, pkgpu::EPI_SWISH, s, g.part, ps && !f.in_g, false, f);   // encoder.c:193-196
-        if (!r) r = gemm(e, w2, h, R, x, b2, pkgpu::EPI_HALF_RESIDUAL, s, g.part, false, false, o);   // encoder.c:198-216
+        if (!r) r = gemm(e, w1, A, R, h, b1, pkgpu::EPI_SWISH, s, &g, ps && !f.in_g, f);   // encoder.c:193-196
+        if (!r) r = gemm(e, w2, h, R, x, b2, pkgpu::EPI_HALF_RESIDUAL, s, &g, false, o);   // encoder.c:198-216
         return r;
     };
     // self-attention (encoder.c:300-424)
@@ -691,7 +691,7 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
         const FusedLn f = fused_in(b.qkv, b.ln_sa_w, b.ln_sa_b, h, b.qkv_b, pkgpu::EPI_NONE);
         const float* A = nullptr;
         int rc = norm_in(f, b.ln_sa_w, b.ln_sa_b, &A, ff1_o.next_g != nullptr);
-        if (!rc) rc = gemm(e, b.qkv, A, R, h, b.qkv_b, pkgpu::EPI_NONE, s, g.part, ps && !f.in_g, false, f);
+        if (!rc) rc = gemm(e, b.qkv, A, R, h, b.qkv_b, pkgpu::EPI_NONE, s, &g, ps && !f.in_g, f);
         if (rc) return rc;
         // every chunk of the group in one launch, each with its own length
         double flops = 0.0, bytes = 4.0 * (2 * Tmax - 1) * kD;   // the P rows read
@@ -721,7 +721,7 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
                               : pkgpu::launch_attention(a, g.n, s),
                          "attention");
         });
-        if (!rc) rc = gemm(e, b.out, att, R, x, b.out_b, pkgpu::EPI_RESIDUAL, s, g.part);
+        if (!rc) rc = gemm(e, b.out, att, R, x, b.out_b, pkgpu::EPI_RESIDUAL, s, &g);
         return rc;
     };
     // convolution module (encoder.c:430-476), time-major throughout
@@ -729,7 +729,7 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
         const FusedLn f = fused_in(b.pw1t, b.ln_conv_w, b.ln_conv_b, h, b.pw1_b, pkgpu::EPI_NONE);
         const float* A = nullptr;
         int rc = norm_in(f, b.ln_conv_w, b.ln_conv_b, &A, false);
-        if (!rc) rc = gemm(e, b.pw1t, A, R, h, b.pw1_b, pkgpu::EPI_NONE, s, g.part, ps && !f.in_g, false, f);
+        if (!rc) rc = gemm(e, b.pw1t, A, R, h, b.pw1_b, pkgpu::EPI_NONE, s, &g, ps && !f.in_g, f);
         // The GLU is formed inside the depthwise convolution, as the kernel
         // stages its input window (each value gated once per workgroup, the
         // window's 8 extra times aside): one launch, and one write and read
@@ -754,7 +754,7 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
         rc = timed(e, PK_GPU_STAGE_CONV, 0.0, (glu_in_dw ? 12.0 : 8.0) * R * kD, s, [&] {
             return check(pkgpu::launch_depthwise(d, g.n, s), "depthwise conv");
         });
-        if (!rc) rc = gemm(e, b.pw2t, ln, R, x, b.pw2_b, pkgpu::EPI_RESIDUAL, s, g.part, false, false, pw2_o);
+        if (!rc) rc = gemm(e, b.pw2t, ln, R, x, b.pw2_b, pkgpu::EPI_RESIDUAL, s, &g, false, pw2_o);
         return rc;
     };
     for (int m = from; m < to; ++m) {
@@ -957,7 +957,7 @@ int run_queued(pk_gpu_encoder* e, const float* x, int T, int chunk, int ov, floa
     // length, with rows relative to the group; the lengths follow at entry
     // rows_cap.
     std::vector<RowGroup> groups = plan_groups(chunks, e->n_groups);
-    e->several_groups = groups.size() > 1;
+    for (RowGroup& g : groups) g.shares_chip = groups.size() > 1;
     std::vector<int> table, lens;
     {
         size_t ci = 0;
@@ -1273,8 +1273,7 @@ int project_positions(pk_gpu_encoder* e, int T)
         fresh.push_back(d);
         // exact chains in every numerics mode: the projections are constants
         // that later runs in any mode read (encoder.c:319-338)
-        rc = gemm(e, b.pos, slice, L, static_cast<float*>(d), nullptr, pkgpu::EPI_NONE, e->stream,
-                  nullptr, false, true);
+        rc = gemm(e, b.pos, slice, L, static_cast<float*>(d), nullptr, pkgpu::EPI_NONE, e->stream, nullptr);
         if (rc) break;
     }
     if (!rc) rc = check(hipStreamSynchronize(e->stream), "position projections");
