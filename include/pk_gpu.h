@@ -213,14 +213,14 @@ int pk_gpu_layer_norm_dev(const float *dx, const float *dgamma, const float *dbe
 int pk_gpu_attention_dev(const float *dqkv, int ldq, const float *dP, int ldp,
                          const float *dpos_bias_u, const float *dpos_bias_v,
                          float *dout, int ldo, int T, int H, void *stream);
-/* Workspace (floats) pk_gpu_attention_ws_dev needs for T rows and H heads:
- * 0 up to T = 512 (the score rows stay on chip), else about H * T^2. */
+/* Workspace (floats) pk_gpu_attention_ws_dev takes for T rows and H heads:
+ * 0 up to T = 512, else about H * T^2. */
 size_t pk_gpu_attention_ws_floats(int T, int H);
 /* pk_gpu_attention_dev for any T (the reference attends over a whole
- * sequence when chunking is off, encoder.c:595-610), the score rows of
- * T > 512 in the caller's 16-byte aligned workspace dws of ws_floats >=
- * pk_gpu_attention_ws_floats(T, H) floats (unused up to 512).  Same
- * operations and bits as pk_gpu_attention_dev. */
+ * sequence when chunking is off, encoder.c:595-610).  T > 512 demands a
+ * 16-byte aligned workspace dws of ws_floats >= pk_gpu_attention_ws_floats(T, H)
+ * floats; the score rows go through it from T = 1345 on and stay on chip below.
+ * Same operations and bits as pk_gpu_attention_dev. */
 int pk_gpu_attention_ws_dev(const float *dqkv, int ldq, const float *dP, int ldp,
                             const float *dpos_bias_u, const float *dpos_bias_v,
                             float *dout, int ldo, int T, int H, float *dws, size_t ws_floats,
@@ -303,11 +303,11 @@ int pk_gpu_encoder_create(pk_gpu_encoder **enc, const pk_gpu_block_weights *bloc
  * reference uses PK_CHUNK_SIZE 400 and PK_CHUNK_OVERLAP 8).  A chunk (or
  * the sequence) of T' frames needs the positional table's rows centre - T' + 1
  * .. centre + T' - 1 (T' <= 5000 for the reference's 9999-row table; longer
- * is PK_GPU_EINVAL).  Chunks up to 512 frames keep attention scores on chip;
- * a longer one (chunking off, as PK_CHUNK=0 runs the reference) keeps them in
- * a workspace of H * T'^2 floats, and the first run that long recomputes every
- * block's position projection for the longer slice.  Host pointers; returns
- * when out is written. */
+ * is PK_GPU_EINVAL).  Attention scores stay on chip up to 1344 frames; a
+ * longer sequence or chunk (chunking off, as PK_CHUNK=0 runs the reference)
+ * keeps them in a workspace of H * T'^2 floats.  The first run of more than
+ * 512 recomputes every block's position projection for the longer slice.
+ * Host pointers; returns when out is written. */
 int pk_gpu_encoder_run(pk_gpu_encoder *enc, const float *x, int T, int chunk_size,
                        int overlap, float *out);
 /* The same with device pointers, enqueued on `stream` (NULL = HIP's null

@@ -7,14 +7,13 @@
 
 namespace pkgpu {
 
-// Longest chunk that attends without a workspace.  The reference's encoder
-// never attends over more than 500 frames unless chunking is forced off
-// (PK_CHUNK_THRESHOLD, parakeet.h; encoder.c:595-610); for longer sequences the
-// caller gives AttnArgs::scores, which holds the score rows that LDS does not.
+// Longest chunk of the fast attention, and of pk_gpu_attention_dev, which takes
+// no workspace.  The reference's encoder never attends over more than 500 frames
+// unless chunking is forced off (PK_CHUNK_THRESHOLD, parakeet.h;
+// encoder.c:595-610).
 constexpr int kAttnMaxT = 512;
 constexpr int kAttnRows = 32;          // query rows per workgroup (fast and long)
-// Row stride of a workgroup's score rows in that workspace, and in the fast
-// attention's LDS.
+// Row stride of a workgroup's score rows in AttnArgs::scores.
 __host__ __device__ constexpr int attn_sld(int T) { return ((T + 31) & ~31) + 8; }
 // Row stride of the exact attention's score rows in LDS: 4 more than a multiple
 // of 32 floats, so that the 4 x 16 scores a wave instruction stores (rows 4
@@ -27,6 +26,9 @@ constexpr size_t attn_lds_bytes(int T, int rt, int nw, bool stage)
 {
     return 4u * ((stage ? (size_t)(rt + nw) * 16 * 132 : 0) + (size_t)16 * rt * attn4_sld(T));
 }
+// Whether the exact attention keeps the score rows in LDS (T <= 1344); those of
+// longer sequences go through AttnArgs::scores.
+constexpr bool attn_scores_in_lds(int T) { return attn_lds_bytes(T, 1, 8, true) <= kLdsBytes; }
 
 // Sequences of at most kAttnShortT rows never take the fast attention.
 constexpr int kAttnShortT = 64;
@@ -47,16 +49,19 @@ struct AttnArgs {
     const int* chunk_rows;     // device, n entries (null: one chunk at row 0)
     const int* chunk_T;        // device, n entries, each in [1, T] (null: all T)
     int T, H;
-    // T > kAttnMaxT: attn_scores_floats(T, H, n) floats of device workspace,
-    // one slice of score rows per workgroup (unused otherwise)
+    // unless attn_scores_in_lds(T): attn_score_rows_floats(T, H, n) floats of
+    // device workspace, one slice of score rows per workgroup
     float* scores;
 };
-// Workspace floats the attention of n chunks of up to T rows needs (0 when
-// its score rows fit in LDS).
+// Floats of all score rows of n chunks of up to T rows.
+inline size_t attn_score_rows_floats(int T, int H, int n_chunks)
+{
+    return (size_t)((T + kAttnRows - 1) / kAttnRows) * H * n_chunks * kAttnRows * attn_sld(T);
+}
+// Workspace floats the exact attention of them reads.
 inline size_t attn_scores_floats(int T, int H, int n_chunks)
 {
-    if (T <= kAttnMaxT) return 0;
-    return (size_t)((T + kAttnRows - 1) / kAttnRows) * H * n_chunks * kAttnRows * attn_sld(T);
+    return attn_scores_in_lds(T) ? 0 : attn_score_rows_floats(T, H, n_chunks);
 }
 
 // Depthwise convolution over time with optional Swish (tensor_ops.c:476-548,

@@ -1795,8 +1795,8 @@ hipError_t run_attention4(const AttnArgs& a, int n_chunks, hipStream_t s)
 hipError_t launch_attention(const AttnArgs& a, int n_chunks, hipStream_t s)
 {
     if (a.T <= 0 || n_chunks <= 0) return hipSuccess;
-    if (a.T > kAttnMaxT && !a.scores) return hipErrorInvalidValue;      // attn_scores_floats asks for it
-    if (attn_lds_bytes(a.T, 1, 8, true) > kLdsBytes) {
+    if (!attn_scores_in_lds(a.T)) {
+        if (!a.scores) return hipErrorInvalidValue;                     // attn_scores_floats asks for it
         const dim3 grid((a.T + kAttnRows - 1) / kAttnRows, a.H, n_chunks);
         if ((size_t)grid.x * grid.y * grid.z * kAttnRows * attn_sld(a.T) >= ((size_t)1 << 40))
             return hipErrorInvalidValue;

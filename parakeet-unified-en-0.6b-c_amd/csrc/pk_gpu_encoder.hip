@@ -76,7 +76,7 @@ struct Chunk {
 struct RowGroup {
     int r0 = 0, R = 0, Tmax = 0, tab = 0, n = 0;
     std::map<int, std::pair<int, int>> by_len;
-    size_t scores_off = 0;      // its attention's score rows (Tmax > kAttnMaxT) in e->scores
+    size_t scores_off = 0;      // its attention's score rows in e->scores, where LDS does not hold them
     float* part = nullptr;      // its split-K partial tiles (fast numerics), or null
     bool shares_chip = false;   // other groups of the run replay beside it
 };
@@ -116,7 +116,7 @@ struct pk_gpu_encoder {
     size_t ws_rows = 0;
     float *x = nullptr, *ln = nullptr, *h = nullptr, *att = nullptr;
     int* rows_tab = nullptr;            // device: chunk rows [rows_cap], then chunk lengths [rows_cap]
-    float* scores = nullptr;            // attention score rows of sequences beyond kAttnMaxT
+    float* scores = nullptr;            // attention score rows that LDS does not hold
     size_t scores_n = 0;                // floats
     size_t rows_cap = 0;
     std::vector<int> tab_host;          // what rows_tab was last given (kept alive for the copy)
@@ -708,7 +708,7 @@ int run_block(pk_gpu_encoder* e, const DevBlock& b, const RowGroup& g, hipStream
         a.chunk_rows = rows;
         a.chunk_T = lens;
         a.T = Tmax; a.H = kHeads;
-        a.scores = Tmax > pkgpu::kAttnMaxT ? e->scores + g.scores_off : nullptr;
+        a.scores = pkgpu::attn_scores_in_lds(Tmax) ? nullptr : e->scores + g.scores_off;
         // Fast numerics: split bf16 operands, prepared in the row group's
         // split-K workspace, which nothing holds between the QKV GEMM (K is
         // not split for it) and the output projection.
@@ -1588,7 +1588,7 @@ int attention_call(const float* dqkv, int ldq, const float* dP, int ldp, const f
     if (!dqkv || !dP || !dpu || !dpv || !dout) return error(PK_GPU_EINVAL, "NULL operand");
     if ((reinterpret_cast<uintptr_t>(dqkv) | reinterpret_cast<uintptr_t>(dP)) % 16)
         return error(PK_GPU_EINVAL, "qkv and P must be 16-byte aligned");
-    const size_t need = pkgpu::attn_scores_floats(T, H, 1);
+    const size_t need = pk_gpu_attention_ws_floats(T, H);
     if (need && (!dws || ws_floats < need || reinterpret_cast<uintptr_t>(dws) % 16))
         return error(PK_GPU_EINVAL, "T = %d needs a 16-byte aligned workspace of %zu floats "
                      "(pk_gpu_attention_ws_floats)", T, need);
@@ -1617,7 +1617,9 @@ int pk_gpu_attention_dev(const float* dqkv, int ldq, const float* dP, int ldp, c
 
 size_t pk_gpu_attention_ws_floats(int T, int H)
 {
-    return T < 1 || H < 1 ? 0 : pkgpu::attn_scores_floats(T, H, 1);
+    // from kAttnMaxT on, where no kernel needs it up to attn_scores_in_lds too:
+    // what callers of any build have to bring
+    return T <= pkgpu::kAttnMaxT || H < 1 ? 0 : pkgpu::attn_score_rows_floats(T, H, 1);
 }
 
 int pk_gpu_attention_ws_dev(const float* dqkv, int ldq, const float* dP, int ldp, const float* dpu,

@@ -3,14 +3,17 @@
 The reference attends over the whole sequence when chunking is off
 (PK_CHUNK=0, encoder.c:595-610; T up to the positional table's 5000 rows,
 workspace encoder.c:49-85).  The attention kernel keeps score rows in LDS up
-to 512 frames; beyond that each workgroup's score rows live in a device
-workspace and the same operations run in the same order, and every block's
-position projection is recomputed once for the longer positional slice.
+to 1344 frames; beyond that each workgroup's score rows live in a device
+workspace and the same operations run in the same order.  Past 512 frames every
+block's position projection is recomputed once for the longer positional slice.
 Each output must equal the oracle's whole encoder (pk_oracle_encoder.c, the
 reference's order of operations) bit for bit:
-  600 frames, 2 blocks   T % 8 == 0, just past the LDS limit
+  600 frames, 2 blocks   T % 8 == 0, just past the projections made at creation
   1100 frames, 1 block   T % 8 == 4: softmax's scalar tail
+  1348 frames, 1 block   just past LDS, T % 8 == 4
   5000 frames, 1 block   the longest sequence the table allows
+  2790 frames, chunks of 1100, 1500, 1500 and 1090 rows, one and two row groups:
+  score rows of several chunks, of their own lengths, in each group's slice
 and after a long run, shorter and chunked runs on the same encoder still
 match (the projections and graphs were replaced, not mixed)."""
 import ctypes
@@ -68,7 +71,7 @@ def features(T, tag):
     return bench.enc_rng(0xFEA7, tag).standard_normal((T, bench.D)).astype(np.float32)
 
 
-@pytest.mark.parametrize("T,n_blocks", [(600, 2), (1100, 1), (5000, 1)])
+@pytest.mark.parametrize("T,n_blocks", [(600, 2), (1100, 1), (1348, 1), (5000, 1)])
 def test_unchunked_long_sequence_bit_exact(model, T, n_blocks):
     x = features(T, 7)
     want = po.encoder(model.blocks, n_blocks, model.pe, bench.PE_CENTER, x, 0, 0)
@@ -78,6 +81,42 @@ def test_unchunked_long_sequence_bit_exact(model, T, n_blocks):
             assert bits_equal(got, want), f"run {i}: {describe_mismatch(got, want)}"
     finally:
         enc.close()
+
+
+@pytest.mark.parametrize("n_groups", [1, 2])
+def test_chunks_past_lds_bit_exact(model, n_groups):
+    """Chunks of unequal lengths, some past the LDS limit and some not, in one
+    attention launch per row group."""
+    T, chunk, ov = 2790, 700, 400
+    lens = [min(o + chunk + ov, T) - max(o - ov, 0) for o in range(0, T, chunk)]
+    assert min(lens) < 1344 < max(lens) and len(set(lens)) > 2
+    x = features(T, 13)
+    want = po.encoder(model.blocks, 1, model.pe, bench.PE_CENTER, x, chunk, ov)
+    enc = Encoder(model, 1)
+    try:
+        pk.call("pk_gpu_encoder_set_groups", enc.enc, n_groups)
+        for i, got in enumerate(enc.run(x, chunk, ov)):
+            assert bits_equal(got, want), f"run {i}: {describe_mismatch(got, want)}"
+    finally:
+        enc.close()
+
+
+def test_score_rows_take_memory_only_past_lds(model):
+    """What an encoder holds after an unchunked run: the position projections of
+    the longer slice, the activations of its rows, and the score rows where LDS
+    does not hold them."""
+    lib, D = pk.load(), bench.D
+    for T, sld in ((1100, 0), (1344, 0), (1348, 1384)):
+        enc = Encoder(model, 1)
+        try:
+            made = lib.pk_gpu_encoder_bytes(enc.enc)
+            enc.run(features(T, 17), 0, 0, reps=1)
+            slice_T = (T + 63) // 64 * 64
+            grown = 4 * D * 2 * (slice_T - 512) + 4 * T * (3 * D + bench.FF)
+            scores = 4 * ((T + 31) // 32 * 32) * 8 * sld
+            assert lib.pk_gpu_encoder_bytes(enc.enc) - made == grown + scores, T
+        finally:
+            enc.close()
 
 
 def test_long_then_short_and_chunked(model):
@@ -115,11 +154,11 @@ def trained_like():
     return m
 
 
-@pytest.mark.parametrize("T,n_blocks", [(1100, 1), (640, 2)])
+@pytest.mark.parametrize("T,n_blocks", [(1100, 1), (640, 2), (1348, 1)])
 def test_unchunked_long_sequence_fast_numerics(trained_like, T, n_blocks):
-    """PK_GPU_NUMERICS_FAST on sequences past the LDS attention limit: the
-    weight GEMMs (M = T) take the split kernels, attention keeps its exact
-    workspace path.  With trained-like attention weights the output stays
+    """PK_GPU_NUMERICS_FAST on sequences past the fast attention's limit: the
+    weight GEMMs (M = T) take the split kernels, attention its exact kernels,
+    with the scores in LDS (640, 1100) and in the workspace (1348).  With trained-like attention weights the output stays
     within 1e-3 of the oracle's exact encoder (the split GEMMs are within
     about 1e-5 each), and a replay repeats the first run bit for bit."""
     model = trained_like
