@@ -576,11 +576,12 @@ int pk_gpu_force_config(int index);
 
 /* The exact GEMMs' own tiles (16-byte aligned rows, alpha = 1): their number,
  * the one that a shape with weights of `bits` = 4, 8 or 32 bits takes (-1:
- * invalid), and a test hook that forces one for later GEMM calls on this
+ * invalid; _shared: in an encoder whose row groups replay side by side), and a test hook that forces one for later GEMM calls on this
  * thread (-1 = automatic).  The tile never changes a result.  A resident
  * encoder keeps a graph per forced tile, as for pk_gpu_force_config. */
 int pk_gpu_num_chain_tiles(void);
 int pk_gpu_pick_chain_tile(int M, int N, int K, int bits);
+int pk_gpu_pick_chain_tile_shared(int M, int N, int K, int bits);
 int pk_gpu_force_chain_tile(int tile);
 
 #ifdef __cplusplus

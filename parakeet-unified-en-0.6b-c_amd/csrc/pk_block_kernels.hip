@@ -207,8 +207,9 @@ __global__ __launch_bounds__(256) void layer_norm_split_rows(const float* x, int
 // block 0's A broadcast to all 16 blocks (CBSZ = 4): one MFMA = 4 rows x 64
 // columns, lane j holds column j of rows 0..3, and the A register lane 4t + i
 // holds row i at k-step t (ABID = t).  Measured, one sequence of 8 heads, us,
-// against the latter (with its scores in LDS up to T = 512): T = 33 9.0 -> 8.6,
-// 100 20.4 -> 12.3, 416 48.4 -> 23.5, 700 99.9 -> 58.1, 1101 220.7 -> 142.
+// against the latter (with its scores in LDS up to T = 512): T = 33 8.9 -> 8.5,
+// 100 20.1 -> 12.0, 416 48.4 -> 22.6, 700 99.5 -> 57.4, 1101 220.7 -> 141.6, 1344
+// 265 -> 164.
 //
 // Scores (NT dot products, blas.c:221-249): eight accumulators per output,
 // step k goes to accumulator k % 8, so accumulator l is the chain over
@@ -1559,8 +1560,9 @@ constexpr int kSub = 256;          // PK_SUB_CHANNELS
 // largest array of the pre-encode (839 MB for 25600 frames, 178 us to write at
 // the chip's copy rate and as much to read back), so it stays in registers: a
 // thread is one channel and keeps three columns of 2 kFcRows + 1 conv.0 values, a
-// workgroup produces kFcRows x kFcCols outputs of conv.2.  Neighbouring rows of
-// workgroups both compute the conv.0 row between them (1/9 more work).  Every
+// workgroup produces kFcRows x kFcCols outputs of conv.2.  Neighbouring
+// workgroups both compute the conv.0 row or column between them (9 rows for 8 and
+// 17 columns for 16: a fifth more work).  Every
 // output is the same chain as from memory.  Bound by its VALU instructions
 // (about 60 per output); 25600 frames: 555 us as two kernels, 92 as this one.
 //
@@ -1784,11 +1786,11 @@ hipError_t run_attention4(const AttnArgs& a, int n_chunks, hipStream_t s)
 
 // Which attention kernel: by the workgroups that 16 and 32 query rows a
 // workgroup make of the launch (us, one sequence of 8 heads unless said):
-// - up to one 16-row workgroup a CU, its operands staged: 23.5 at T = 416, where
-//   32 rows, unstaged, take 39.4; also beyond T = 1024, where 32 rows' scores
+// - up to one 16-row workgroup a CU, its operands staged: 22.6 at T = 416, where
+//   32 rows, unstaged, take 39.8; also beyond T = 1024, where 32 rows' scores
 //   leave one workgroup a CU (142 against 158 at T = 1101);
-// - up to one 32-row workgroup a CU: 8 waves, unstaged: 58.5 at T = 700 (16 rows
-//   staged 66.2, 32 rows by 4 waves 63.2);
+// - up to one 32-row workgroup a CU: 8 waves, unstaged: 57.4 at T = 700 (16 rows
+//   staged 65.9, 32 rows by 4 waves 62.2);
 // - more (an encoder's chunks): 4 waves, unstaged, two workgroups a CU: exact
 //   encoder at 3200 frames 37.6 ms (8 waves 38.4, 16 rows staged 38.2);
 // - scores that do not fit in LDS: rel_pos_attention_long.

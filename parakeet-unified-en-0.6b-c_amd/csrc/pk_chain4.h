@@ -100,10 +100,12 @@ struct Tile {
     static constexpr int NT = 64 * NP;                // staging threads
     static constexpr int BM = 16 * R * NWM, BN = 16 * C * NWN;
     // Rows (of A, and columns of W) are S floats apart in LDS, and W has 4
-    // more floats after every 8 columns.  With 32 banks of 4 bytes, b128
-    // accesses of 8 lanes and b32 ones of 32 a cycle, the operand reads (8
+    // more floats after every 8 columns.  Laid out for 32 banks of 4 bytes, b128
+    // accesses of 8 lanes and b32 ones of 32 a cycle: the operand reads (8
     // rows, one group) and both kinds of stores (4 rows x 8 units of A; 8
-    // units of W at 4 steps k, k + 4, ...) each touch every bank once.
+    // units of W at 4 steps k, k + 4, ...) then each touch every bank once.
+    // The counter still reads 0.33 conflict cycles for each cycle of LDS work,
+    // in every tile and format, which is 0.16 to 0.37 of a launch's.
     static constexpr int S = KT + 4;
     static constexpr int A_LDS = BM * S, B_LDS = BN * S + BN / 2, BUF = A_LDS + B_LDS;
     static constexpr int NQ = BN / 8, NQL = NQ < 8 ? NQ : 8, K16 = KT / 16;

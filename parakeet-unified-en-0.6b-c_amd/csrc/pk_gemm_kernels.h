@@ -210,8 +210,9 @@ enum Tolerance { TOL_NONE = 0, TOL_SMALL_M = 1, TOL_ALL = 2 };
 
 // Launch the whole GEMM (beta pre-pass semantics, early exits, int8 edge
 // columns) on `stream`.  Returns hipSuccess or the launch error.
-// cfg_index < 0 selects choose_config_index(); a forced configuration
-// (cfg_index >= 0) always runs the exact chains.
+// cfg_index < 0: the exact chains take a four-deep tile (pk_chain4.h), or
+// choose_config_index() where those do not apply; a forced configuration
+// (cfg_index >= 0) always runs its K = 1 chains.
 hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream, int cfg_index,
                        Tolerance tol = TOL_NONE);
 

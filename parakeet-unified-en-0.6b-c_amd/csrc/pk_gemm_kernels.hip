@@ -64,8 +64,10 @@ int num_configs() { return kNumConfigs; }
 TileConfig config_at(int i) { return kConfigs[i]; }
 
 // Every output is a chain of K dependent MFMA steps, so the work that can run
-// at once is the number of independent chains (M*N / outputs per MFMA).
-// Chosen from a sweep of every configuration over the encoder's GEMM shapes
+// at once is the number of independent chains (M*N / outputs per MFMA).  The
+// encoder's GEMMs take the four-deep tiles (chain4_pick); what comes here has
+// alpha other than 1 or operands without vector loads, at any of these sizes.
+// Chosen, while the encoder's GEMMs ran here, from a sweep of every configuration over the encoder's GEMM shapes
 // on MI355X (hot weights; times in us for the best and the chosen config):
 //   M*N < 200K          config 12 (S 4x4, 1 chain)    QKV M=32: 11.6
 //   M*N < 1M, K >= 2048 config 17 (S 4x4, 8+8 waves)  FF down M=375: 51.6
@@ -90,7 +92,7 @@ static int choose_index(int M, int N, int K, WeightKind kind = W_I8)
     if (outputs < 1.0e6) return K >= 2048 ? 17 : 13;
     if (outputs < 1.6e6) return 14;
     if (outputs < 3.0e6) return 18;
-    // Long M (the encoder's batched chunks): measured per weight format at
+    // Long M: measured per weight format, on the encoder's batched chunks, at
     // M = 3312, and for the int4 projections also at M = 1656 (one of two
     // row groups whose kernels run side by side).  Two LDS chunks in flight
     // (fewer registers, 3 waves per SIMD) win except for the int4 down
@@ -127,9 +129,12 @@ namespace {
 // on 64 x 64, K = 1 391; 204800 x 256 x 256 int4: 332, 240, 266).
 //
 // shares_chip: other kernels run beside the GEMM and take what its last round
-// leaves free, so a part of a round counts as that part; and 128 x 64 tiles, one
-// workgroup of whose registers fill a CU, are left out.  3200 frames in two row
-// groups: 38.2 ms with each GEMM's own best tile, 37.1 so (37.9 with 128 x 64).
+// leaves free, so a part of a round counts as that part; and 128 x 64 tiles are
+// left out.  That is measured, its cause is not: two of their workgroups fit a CU
+// (86 registers, 55.5 KB of LDS), of the others three or more.  Exact encoder in
+// two row groups, one box, ms at 1600 / 2400 / 3200 / 4800 / 6400 frames: 20.7 /
+// 31.4 / 37.7 / 52.5 / 69.5; with 128 x 64 20.8 / 31.8 / 38.4 / 54.7 / 68.9; with
+// each GEMM's own best tile 21.5 / 30.2 / 40.0 / 55.5 / 72.3.
 struct Rounds { float a, b, e, c, e0; };
 constexpr Rounds kChain4Rounds[3][chain4::kNumTiles] = {
     /* fp32 */ {{2.9f, 3.9f, 0.1f, 3.75f, 0.76f}, {2.8f, 4.3f, 0.2f, 4.0f, 0.65f},
@@ -147,7 +152,7 @@ constexpr int kCus = 256;
 constexpr double kL2BytesPerUs = 12e6;
 thread_local int t_chain_tile = -1;
 
-int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip = false)
+int chain4_pick(int M, int N, int K, WeightKind kind, bool shares_chip)
 {
     const double k = K / 1024.0;
     const double w_bytes = (kind == W_F32 ? 4.0 : kind == W_I8 ? 1.0 : 0.625) * K * N;
@@ -373,20 +378,24 @@ hipError_t launch_swish(const float* x, float* y, long long n, hipStream_t strea
 
 }  // namespace pkgpu
 
+static int pick_tile(int M, int N, int K, int bits, bool shares_chip)
+{
+    if (M <= 0 || N <= 0 || K <= 0) return -1;
+    switch (bits) {
+    case 4: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I4, shares_chip);
+    case 8: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I8, shares_chip);
+    case 32: return pkgpu::chain4_pick(M, N, K, pkgpu::W_F32, shares_chip);
+    default: return -1;
+    }
+}
+
 extern "C" {
 
 int pk_gpu_num_chain_tiles(void) { return pkgpu::chain4::kNumTiles; }
 
-int pk_gpu_pick_chain_tile(int M, int N, int K, int bits)
-{
-    if (M <= 0 || N <= 0 || K <= 0) return -1;
-    switch (bits) {
-    case 4: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I4);
-    case 8: return pkgpu::chain4_pick(M, N, K, pkgpu::W_I8);
-    case 32: return pkgpu::chain4_pick(M, N, K, pkgpu::W_F32);
-    default: return -1;
-    }
-}
+int pk_gpu_pick_chain_tile(int M, int N, int K, int bits) { return pick_tile(M, N, K, bits, false); }
+
+int pk_gpu_pick_chain_tile_shared(int M, int N, int K, int bits) { return pick_tile(M, N, K, bits, true); }
 
 int pk_gpu_force_chain_tile(int tile)
 {

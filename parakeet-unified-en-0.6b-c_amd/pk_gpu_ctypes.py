@@ -48,6 +48,7 @@ _PROTOS = {
     "pk_gpu_encoder_graphs": (_i, [_p]),
     "pk_gpu_num_chain_tiles": (_i, []),
     "pk_gpu_pick_chain_tile": (_i, [_i, _i, _i, _i]),
+    "pk_gpu_pick_chain_tile_shared": (_i, [_i, _i, _i, _i]),
     "pk_gpu_force_chain_tile": (_i, [_i]),
     "pk_gpu_set_numerics": (_i, [_i]),
     "pk_gpu_get_numerics": (_i, []),

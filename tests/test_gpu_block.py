@@ -76,8 +76,9 @@ def gpu_attention(dev, qkv, P, pu, pv):
 
 @pytest.mark.parametrize("T", [416, 408, 64, 24, 8, 1, 21, 108, 300, 512, 33, 17, 49, 50, 63, 65])
 def test_attention_bit_exact_to_oracle(dev, T):
-    """T <= 64 takes the short-sequence kernel (every row staged in LDS at
-    once; one or two blocks of positions: T = 49 / 50), longer T the tiled one."""
+    """Lengths around the tiles of 16 rows and the softmax's groups of 8, one
+    sequence of 8 heads (16 query rows a workgroup; the other forms:
+    test_gpu_attention4.py)."""
     qkv, P, pu, pv = attention_inputs(T)
     got = gpu_attention(dev, qkv, P, pu, pv)
     want = po.attention_core(qkv, P, pu, pv)
@@ -98,8 +99,9 @@ def test_attention_bit_exact_to_reference(dev, T):
 
 @pytest.mark.parametrize("T", [513, 640, 1000])
 def test_attention_long_sequence_bit_exact_to_oracle(dev, T):
-    """Past 512 rows the score rows live in the caller's workspace: the same
-    bits as the oracle (T = 1000: softmax's scalar tail)."""
+    """Past 512 rows the caller brings a workspace, whatever the kernel does
+    with it: the same bits as the oracle (513: softmax's scalar tail), and a
+    workspace too small is refused."""
     lib = pk.load()
     qkv, P, pu, pv = attention_inputs(T)
     D = bg.H * bg.DH
@@ -234,8 +236,8 @@ def test_encoder_weight_directories_bit_exact_to_oracle(dev, mode, T, chunk):
     fp32: QKV, position and output projections on the fp32 chains), two
     blocks, bit for bit against the oracle's encoder on the same blocks: an
     unchunked 300-frame sequence (softmax's scalar tail), 64-frame chunks
-    of 72, 76 and 12 rows, and 40-frame chunks of 48, 56 and 28 rows (the
-    short-sequence attention over a batch of chunks)."""
+    of 72, 76 and 12 rows, and 40-frame chunks of 48, 56 and 28 rows (short
+    chunks in one attention launch)."""
     blocks = [bg.Block(0xD1500 + i, attn_scale=0.0005, mode=mode) for i in range(2)]
     assert {blocks[0].w.ff1_linear1_w.bits, blocks[0].w.linear_out_w.bits} == \
         {8 if mode == "int8" else 32}

@@ -87,9 +87,10 @@ def test_tile_configs_are_well_formed():
         assert 0 <= lib.pk_gpu_pick_config(*shape) < len(cfgs)
 
 
-# The encoder's GEMMs at 3200 frames: one row group (M = 3312) and each of two
-# row groups (M = 1656).  These picks were measured on the encoder itself;
-# a change to the dispatcher that moves one of them needs a new measurement.
+# The K = 1 chain kernels' picks for the shapes of the encoder's GEMMs at 3200
+# frames, where they were measured while the encoder's GEMMs ran on them.  They
+# serve GEMMs of any size with alpha other than 1 or unaligned operands; the
+# encoder's own take the four-deep tiles below.
 ENCODER_PICKS = [
     # bits, M, N, K, config
     (4, 3312, 4096, 1024, 20), (4, 3312, 1024, 4096, 11),
@@ -105,6 +106,44 @@ ENCODER_PICKS = [
 @pytest.mark.parametrize("bits,M,N,K,cfg", ENCODER_PICKS)
 def test_dispatcher_picks_for_encoder_shapes(bits, M, N, K, cfg):
     assert pk.load().pk_gpu_pick_config_bits(M, N, K, bits) == cfg
+
+
+# The four-deep tiles of the encoder's GEMMs at 3200 frames: one row group (M =
+# 3312, alone on the chip) and each of two side by side (M = 1656), and of the
+# feed-forward pairs of 375 and 500 rows.  Measured on the encoder and the pairs:
+# a change to the rule that moves one of them needs a new measurement.
+CHAIN_PICKS = [
+    # bits, M, N, K, tile alone, tile beside another row group
+    (4, 3312, 4096, 1024, 4, 4), (4, 3312, 1024, 4096, 3, 4),
+    (4, 1656, 4096, 1024, 3, 4), (4, 1656, 1024, 4096, 5, 4),
+    (8, 3312, 3072, 1024, 5, 4), (8, 3312, 1024, 1024, 1, 4),
+    (8, 1656, 3072, 1024, 4, 4), (8, 1656, 1024, 1024, 1, 4),
+    (32, 3312, 2048, 1024, 3, 4), (32, 3312, 1024, 1024, 3, 4),
+    (32, 1656, 2048, 1024, 3, 4), (32, 1656, 1024, 1024, 4, 3),
+    (4, 375, 4096, 1024, 3, 4), (4, 375, 1024, 4096, 2, 2),
+    (32, 500, 4096, 1024, 4, 4), (32, 500, 1024, 4096, 3, 3),
+]
+
+
+@pytest.mark.parametrize("bits,M,N,K,alone,shared", CHAIN_PICKS)
+def test_chain_tile_picks_for_encoder_shapes(bits, M, N, K, alone, shared):
+    lib = pk.load()
+    assert lib.pk_gpu_pick_chain_tile(M, N, K, bits) == alone
+    assert lib.pk_gpu_pick_chain_tile_shared(M, N, K, bits) == shared
+
+
+def test_chain_tile_choice_beside_other_kernels():
+    """Beside other kernels the 128 x 64 tile is never taken while another one's
+    rows fit the grid."""
+    lib = pk.load()
+    for bits in (4, 8, 32):
+        for N in (256, 1024, 4096):
+            for M in (16, 375, 1656, 3312, 25600, 64 * 65535):
+                for K in (256, 1024, 4096):
+                    assert 0 <= lib.pk_gpu_pick_chain_tile_shared(M, N, K, bits) < 5
+    assert lib.pk_gpu_pick_chain_tile_shared(64 * 65535 + 1, 256, 256, 32) == 5
+    assert lib.pk_gpu_pick_chain_tile_shared(16, 16, 16, 7) == -1
+    assert lib.pk_gpu_pick_chain_tile_shared(16, 16, 0, 8) == -1
 
 
 def test_epilogue_validation_precedes_device_use():
